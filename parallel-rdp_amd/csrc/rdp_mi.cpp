@@ -262,6 +262,7 @@ struct Context : Lane {
 	std::mutex lock;
 	uint8_t *d_digest = nullptr;                // rdp_mi_state_digest: one target and its result
 	DeviceBuffer view;                          // rdp_mi_framebuffer_view output
+	ViStaging vi_stage;                         // image of a waiting scanout
 
 	int init()
 	{
@@ -2384,7 +2385,8 @@ static int scanout_queue(Processor &p, const rdp_mi_scanout_options &opts, uint3
 	src.hplanes = p.d_up_hidden;
 	src.rdram = p.up_log2 ? p.d_up_rdram : p.d_rdram;
 	src.hidden = p.up_log2 ? p.d_up_hidden : p.d_hidden;
-	int err = vi_scanout(p.vi, p.vi_regs, src, c.d_gamma, c.stream, opts, out, width, height, done == nullptr);
+	int err = vi_scanout(p.vi, p.vi_regs, src, c.d_gamma, c.stream, opts, out, width, height,
+	                     done ? nullptr : &c.vi_stage);
 	if (err) return set_error(err, "VI scanout failed");
 	if (done) HIP_CHECK(hipEventRecord(done, c.stream));
 	return 0;

@@ -1,17 +1,20 @@
-// Video interface scanout: host register decode + two gfx950 kernels.
+// Video interface scanout: host register decode + one gfx950 kernel.
 //
-//   k_vi_filter  one lane per texel of the fetch-filter image: extracts the
-//                VRAM pixels it needs straight from RDRAM (extract_vram.comp)
-//                and applies the AA or dither reconstruction filter
-//                (vi_fetch.frag), writing the normal and the fetch-bug layer.
-//   k_vi_scale   one lane per output pixel: HStart/VStart scissor and
-//                serrate selection, divot median (vi_divot.frag) on the fly
-//                from the filter image, bilinear resampling, gamma / gamma
-//                dither (vi_scale.frag) and the blend with the previous frame
-//                (vi_blend_fields.frag).
+//   k_vi  one wave per 64 output pixels of one line.  The wave first builds the
+//         filter texels its pixels sample (one or two rows of the fetch-filter
+//         image, in LDS): VRAM pixels straight from RDRAM (extract_vram.comp)
+//         through the AA or dither reconstruction filter (vi_fetch.frag).  Then
+//         one lane per output pixel: HStart/VStart scissor and serrate
+//         selection, divot median (vi_divot.frag), bilinear resampling, gamma /
+//         gamma dither (vi_scale.frag) and the blend with the previous frame
+//         (vi_blend_fields.frag).  The pixel goes to the device image (the next
+//         scanout's previous frame) and straight to the host's pinned memory.
 //
-// Images are small (at most ~2600 x 1200 filter texels, 640 x 576 output),
-// so both kernels are bound by launch and L2 latency, not HBM.
+// One kernel instead of a filter image in memory and a second pass over it:
+// only the rows a line samples are filtered (a 480-line frame shown on 240 lines
+// samples every second row with a zero vertical fraction), and nothing waits
+// for a second launch or for a copy engine.  What bounds it is the PCIe write
+// of the image (50 GB/s); natively the rest is launch latency.
 #include "rdp_vi.hpp"
 
 #include <vector>
@@ -109,18 +112,33 @@ void ViState::end_per_scanline()
 
 void ViState::release()
 {
-	if (params_done) {
-		if (params_busy) (void)hipEventSynchronize(params_done);
-		(void)hipEventDestroy(params_done);
-		params_done = nullptr;
-		params_busy = false;
+	if (lines_done) {
+		if (lines_busy) (void)hipEventSynchronize(lines_done);
+		(void)hipEventDestroy(lines_done);
+		lines_done = nullptr;
+		lines_busy = false;
 	}
 	for (auto &p : d_images)
 		if (p) (void)hipFree(p), p = nullptr;
-	if (d_filter) (void)hipFree(d_filter), d_filter = nullptr;
-	if (d_params) (void)hipFree(d_params), d_params = nullptr;
-	if (h_params) (void)hipHostFree(h_params), h_params = nullptr;
-	filter_words = 0;
+	if (d_lines) (void)hipFree(d_lines), d_lines = nullptr;
+	if (h_lines) (void)hipHostFree(h_lines), h_lines = nullptr;
+}
+
+int ViStaging::reserve(size_t want, size_t bands)
+{
+	while (done.size() < bands) {
+		hipEvent_t ev;
+		if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) return RDP_MI_ERROR_DEVICE;
+		done.push_back(ev);
+	}
+	if (want <= words) return 0;
+	if (pixels && hipHostFree(pixels) != hipSuccess) return RDP_MI_ERROR_DEVICE;
+	pixels = nullptr;
+	words = 0;
+	if (hipHostMalloc((void **)&pixels, want * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess)
+		return RDP_MI_ERROR_OUT_OF_MEMORY;
+	words = want;
+	return 0;
 }
 
 namespace {
@@ -295,48 +313,36 @@ DEV void check_neighbor(const Texel &c, uint32_t lo[3], uint32_t hi[3], uint32_t
 
 DEV int clamp1(int v) { return v < -1 ? -1 : (v > 1 ? 1 : v); }
 
-// vi_fetch.frag:58-163: one texel of both layers.
-__global__ __launch_bounds__(256) void k_vi_filter(const ViParams *__restrict__ params, const uint8_t *__restrict__ rdram,
-                                                  const uint8_t *__restrict__ hidden, uint32_t *__restrict__ out)
+// vi_fetch.frag:58-163: texel (x, y) of the fetch-filter image; bug selects the
+// fetch-bug layer.  Zero outside the image.
+DEV uint32_t filter_texel(const ViParams &P, const uint8_t *__restrict__ rdram, const uint8_t *__restrict__ hidden, int x,
+                          int y, bool bug)
 {
-	const ViParams &P = *params;
-	const int x = (int)(blockIdx.x * 16 + (threadIdx.x & 15));
-	const int y = (int)(blockIdx.y * 16 + (threadIdx.x >> 4));
-	if (x >= P.aw || y >= P.ah) return;
+	if (x < 0 || y < 0 || x >= P.aw || y >= P.ah) return 0;
 	const int px = x + 2, py = y + 2;
 	const Texel mid = ext(P, rdram, hidden, px, py);
 	const uint32_t m[3] = { mid.r, mid.g, mid.b };
-	uint32_t color[3], color_bug[3];
+	uint32_t color[3];
 	if (mid.a != 7) {
 		uint32_t lo[3], hi[3], slo[3], shi[3];
 #pragma unroll
 		for (int i = 0; i < 3; i++) lo[i] = hi[i] = slo[i] = shi[i] = m[i];
 		const Texel lu = ext(P, rdram, hidden, px - 1, py - 1), ru = ext(P, rdram, hidden, px + 1, py - 1);
 		const Texel tl = ext(P, rdram, hidden, px - 2, py), tr = ext(P, rdram, hidden, px + 2, py);
-		const Texel ld = ext(P, rdram, hidden, px - 1, py + 1), rd = ext(P, rdram, hidden, px + 1, py + 1);
+		// The line below; with the fetch bug the current line again.
+		const int dx = bug ? 2 : 1, dy = bug ? 0 : 1;
+		const Texel ld = ext(P, rdram, hidden, px - dx, py + dy), rd = ext(P, rdram, hidden, px + dx, py + dy);
 		check_neighbor(lu, lo, hi, slo, shi);
 		check_neighbor(ru, lo, hi, slo, shi);
 		check_neighbor(tl, lo, hi, slo, shi);
 		check_neighbor(tr, lo, hi, slo, shi);
-		uint32_t lob[3], hib[3], slob[3], shib[3];
-#pragma unroll
-		for (int i = 0; i < 3; i++) {
-			lob[i] = lo[i];
-			hib[i] = hi[i];
-			slob[i] = slo[i];
-			shib[i] = shi[i];
-		}
 		check_neighbor(ld, lo, hi, slo, shi);
 		check_neighbor(rd, lo, hi, slo, shi);
 		if (P.fetch_bug) {
-			check_neighbor(tl, lob, hib, slob, shib);
-			check_neighbor(tr, lob, hib, slob, shib);
 #pragma unroll
 			for (int i = 0; i < 3; i++) {
 				if (m[i] == lo[i]) slo[i] = lo[i];
 				if (m[i] == hi[i]) shi[i] = hi[i];
-				if (m[i] == lob[i]) slob[i] = lob[i];
-				if (m[i] == hib[i]) shib[i] = hib[i];
 			}
 		}
 		const uint32_t coeff = 7u - mid.a;
@@ -344,58 +350,45 @@ __global__ __launch_bounds__(256) void k_vi_filter(const ViParams *__restrict__ 
 		for (int i = 0; i < 3; i++) {
 			const uint32_t off = slo[i] + shi[i] - (m[i] << 1);
 			color[i] = (m[i] + ((off * coeff + 4u) >> 3)) & 0xffu;
-			const uint32_t offb = slob[i] + shib[i] - (m[i] << 1);
-			color_bug[i] = (m[i] + ((offb * coeff + 4u) >> 3)) & 0xffu;
 		}
 	} else if (P.status & VI_DITHER_FILTER) {
-		int tmp[3], acc[3] = { 0, 0, 0 }, accb[3];
+		int tmp[3], acc[3] = { 0, 0, 0 };
 #pragma unroll
 		for (int i = 0; i < 3; i++) tmp[i] = (int)(m[i] >> 3);
+		auto add = [&](int dx, int dy) {
+			const Texel t = ext(P, rdram, hidden, px + dx, py + dy);
+			acc[0] += clamp1((int)(t.r >> 3) - tmp[0]);
+			acc[1] += clamp1((int)(t.g >> 3) - tmp[1]);
+			acc[2] += clamp1((int)(t.b >> 3) - tmp[2]);
+		};
+#pragma unroll
 		for (int dy = -1; dy <= 0; dy++)
-			for (int dx = -1; dx <= 1; dx++) {
-				const Texel t = ext(P, rdram, hidden, px + dx, py + dy);
-				acc[0] += clamp1((int)(t.r >> 3) - tmp[0]);
-				acc[1] += clamp1((int)(t.g >> 3) - tmp[1]);
-				acc[2] += clamp1((int)(t.b >> 3) - tmp[2]);
-			}
 #pragma unroll
-		for (int i = 0; i < 3; i++) accb[i] = acc[i];
-		const Texel a = ext(P, rdram, hidden, px - 1, py + 1), b = ext(P, rdram, hidden, px + 1, py + 1);
-		const Texel c = ext(P, rdram, hidden, px, py + 1);
-		const Texel l = ext(P, rdram, hidden, px - 1, py), rr = ext(P, rdram, hidden, px + 1, py);
-		const uint32_t av[3] = { a.r, a.g, a.b }, bv[3] = { b.r, b.g, b.b }, cv[3] = { c.r, c.g, c.b };
-		const uint32_t lv[3] = { l.r, l.g, l.b }, rv[3] = { rr.r, rr.g, rr.b };
+			for (int dx = -1; dx <= 1; dx++)
+				if (dx || dy) add(dx, dy);  // the pixel itself adds nothing
+		// The line below; with the fetch bug the current line again.
+		const int dy = bug ? 0 : 1;
+		add(-1, dy);
+		add(1, dy);
+		if (!bug) add(0, 1);
+		// An out-of-range value written to an 8-bit UINT attachment keeps its low 8 bits.
 #pragma unroll
-		for (int i = 0; i < 3; i++) {
-			acc[i] += clamp1((int)(av[i] >> 3) - tmp[i]) + clamp1((int)(bv[i] >> 3) - tmp[i]) +
-			          clamp1((int)(cv[i] >> 3) - tmp[i]);
-			accb[i] += clamp1((int)(lv[i] >> 3) - tmp[i]) + clamp1((int)(rv[i] >> 3) - tmp[i]);
-			// An out-of-range value written to an 8-bit UINT attachment keeps its low 8 bits.
-			color[i] = ((m[i] & 0xf8u) + (uint32_t)acc[i]) & 0xffu;
-			color_bug[i] = ((m[i] & 0xf8u) + (uint32_t)accb[i]) & 0xffu;
-		}
+		for (int i = 0; i < 3; i++) color[i] = ((m[i] & 0xf8u) + (uint32_t)acc[i]) & 0xffu;
 	} else {
 #pragma unroll
-		for (int i = 0; i < 3; i++) color[i] = color_bug[i] = m[i];
+		for (int i = 0; i < 3; i++) color[i] = m[i];
 	}
-	const size_t idx = (size_t)y * (size_t)P.aw + (size_t)x;
-	out[idx] = pack(Texel{ color[0], color[1], color[2], mid.a });
-	if (P.fetch_bug) out[(size_t)P.aw * (size_t)P.ah + idx] = pack(Texel{ color_bug[0], color_bug[1], color_bug[2], mid.a });
+	return pack(Texel{ color[0], color[1], color[2], mid.a });
 }
 
-// Filter-image texel with the divot median applied when enabled
-// (vi_divot.frag:54-92); zero outside the image.
-DEV Texel filtered(const ViParams &P, const uint32_t *__restrict__ A, int layer, int x, int y)
+// Filter-image texel x of the row in LDS (texels base ..) with the divot median
+// applied when enabled (vi_divot.frag:54-92); zero outside the image.
+DEV Texel filtered(const ViParams &P, const uint32_t *row, int base, int x, int y)
 {
-	const uint32_t *L = A + (size_t)layer * (size_t)P.aw * (size_t)P.ah;
-	auto at = [&](int xx) -> Texel {
-		if (xx < 0 || y < 0 || xx >= P.aw || y >= P.ah) return Texel{ 0, 0, 0, 0 };
-		return unpack(L[(size_t)y * (size_t)P.aw + (size_t)xx]);
-	};
-	if (!P.divot) return at(x);
+	if (!P.divot) return unpack(row[x - base]);
 	// The divot image is (aw - 3) wide and ah high.
 	if (x < 0 || x >= P.aw - 3 || y < 0 || y >= P.ah) return Texel{ 0, 0, 0, 0 };
-	const Texel l = at(x), m = at(x + 1), r = at(x + 2);
+	const Texel l = unpack(row[x - base]), m = unpack(row[x + 1 - base]), r = unpack(row[x + 2 - base]);
 	if ((l.a & m.a & r.a) == 7) return m;
 	auto med = [](uint32_t a, uint32_t b, uint32_t c) { return umax(umin(a, b), umin(umax(a, b), c)); };
 	return Texel{ med(l.r, m.r, r.r), med(l.g, m.g, r.g), med(l.b, m.b, r.b), m.a };
@@ -417,43 +410,95 @@ DEV uint32_t reseed_noise(uint32_t x, uint32_t y, uint32_t z)
 
 DEV uint32_t vi_lerp(uint32_t a, uint32_t b, uint32_t l) { return (a + (((b - a) * l + 16u) >> 5)) & 0xffu; }
 
-// vi_scale.frag:74-153 plus vi_blend_fields.frag.
-__global__ __launch_bounds__(256) void k_vi_scale(const ViParams *__restrict__ params, const uint32_t *__restrict__ A,
-                                                 const uint8_t *__restrict__ gamma, const uint32_t *__restrict__ prev,
-                                                 uint32_t *__restrict__ out)
+// Texels of one filter row a wave holds: 64 pixels at the largest step (0xfff of
+// 1024 texels each, whatever the upscaling factor: it scales the pixels and
+// the texels alike), the right neighbour of the last one and the two texels
+// right of it the divot median reads: (63 * 4095 + 1023) / 1024 + 1 + 1 + 2 < 260.
+constexpr int kViRowTexels = 260;
+
+// vi_fetch.frag, vi_divot.frag, vi_scale.frag:74-153 and vi_blend_fields.frag for
+// 64 output pixels of one line per wave.  P arrives as a kernel argument;
+// lines is null when every line shows the same registers (P.line, on lines
+// line_lo .. line_hi - 1).  The image goes to `out` and to the host's pinned
+// memory `host`; row0 is the first line of this launch.
+//
+// A waiting scanout of a 640x480 frame on 240 lines (AA, divot, dither filter)
+// takes 46 us, against 105 us for a parameter upload, a filter kernel over all
+// 480 lines, a scale kernel and a copy-engine transfer into pageable memory; into
+// pinned memory 29 us.  The 1.2 MB of 480 lines take 32 us in the kernel (38 GB/s
+// over PCIe), 2560x960 pixels of a 4x frame 220 us (45 GB/s).
+__global__ __launch_bounds__(256) void k_vi(const ViParams P, const ViLine *__restrict__ lines,
+                                            const uint8_t *__restrict__ rdram, const uint8_t *__restrict__ hidden,
+                                            const uint8_t *__restrict__ gamma, const uint32_t *__restrict__ prev,
+                                            uint32_t *__restrict__ out, uint32_t *__restrict__ host, int row0, int row1)
 {
-	const ViParams &P = *params;
-	const int px = (int)(blockIdx.x * 64 + (threadIdx.x & 63));
-	const int py = (int)(blockIdx.y * 4 + (threadIdx.x >> 6));
-	if (px >= P.ow || py >= P.oh) return;
+	__shared__ uint32_t s_rows[4][2][kViRowTexels];
+	const int wave = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
+	const int px0 = (int)blockIdx.x * 64, px = px0 + lane;
+	const int py = row0 + (int)blockIdx.y * 4 + wave;
+	if (py >= row1) return;  // waves of a block share nothing
 	uint32_t result = 0;
-	if (px >= P.draw_x && px < P.draw_x + P.draw_w && py >= P.draw_y && py < P.draw_y + P.draw_h) {
-		int cx = px + P.crop_l, cy = py + P.crop_t;
-		const ViLine li = P.lines[cy >> P.info_y_shift];
-		cy -= P.v_start;
-		if (!(cx < li.h_start_clamp || cx >= li.h_end_clamp || ((cy & P.serrate_mask) != P.serrate_select))) {
-			cx -= li.h_start;
-			cy >>= P.serrate_shift;
+	int cy = py + P.crop_t;
+	const int l = cy >> P.info_y_shift;
+	bool shown = py >= P.draw_y && py < P.draw_y + P.draw_h;
+	ViLine li = P.line;
+	if (!lines)
+		shown = shown && l >= P.line_lo && l < P.line_hi;
+	else if (shown)
+		li = lines[l];
+	cy -= P.v_start;
+	// The pixels of this line inside the drawn rectangle and the line's clamps,
+	// in columns relative to the line's start.
+	const int lo = (P.draw_x > li.h_start_clamp - P.crop_l ? P.draw_x : li.h_start_clamp - P.crop_l);
+	const int hi = (P.draw_x + P.draw_w < li.h_end_clamp - P.crop_l ? P.draw_x + P.draw_w : li.h_end_clamp - P.crop_l);
+	const int first = px0 > lo ? px0 : lo, last = (px0 + 64 < hi ? px0 + 64 : hi) - 1;
+	if (shown && first <= last && (cy & P.serrate_mask) == P.serrate_select) {
+		const int dx = P.crop_l - li.h_start;
+		cy >>= P.serrate_shift;
+		const int y = (cy - li.y_base) * li.y_add + li.y_start;
+		const int by = y >> 10;
+		const bool scale = (P.status & VI_META_SCALE) != 0;
+		const uint32_t yf = scale ? (uint32_t)((y >> 5) & 31) : 0;
+		bool bug = false;
+		if (P.fetch_bug) {
+			const int prev_y = (y - P.init_y_add) >> 10, next_y = (y + P.init_y_add) >> 10;
+			bug = cy != 0 && by == prev_y && by != next_y;
+		}
+		// Filter texels base .. end - 1 of row by and, when the line blends two
+		// rows (a zero fraction leaves the upper one unchanged), of row by + 1.
+		const int base = ((first + dx) * li.x_add + li.x_start) >> 10;
+		const int end = (((last + dx) * li.x_add + li.x_start) >> 10) + (scale ? 2 : 1) + (P.divot ? 2 : 0);
+		for (int i = lane; i < end - base; i += 64) {
+			s_rows[wave][0][i] = filter_texel(P, rdram, hidden, base + i, by, false);
+			if (yf) s_rows[wave][1][i] = filter_texel(P, rdram, hidden, base + i, by + 1, bug);
+		}
+		// Order the wave's LDS writes before its own reads.
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+		if (px >= first && px <= last) {
+			const int cx = px + dx;
 			const uint32_t noise = (P.status & VI_GAMMA_DITHER) ? reseed_noise((uint32_t)cx, (uint32_t)cy, P.frame_count) : 0;
-			const int x = cx * li.x_add + li.x_start;
-			const int y = (cy - li.y_base) * li.y_add + li.y_start;
-			const int bx = x >> 10, by = y >> 10;
-			const Texel t00 = filtered(P, A, 0, bx, by);
+			const int x = cx * li.x_add + li.x_start, bx = x >> 10;
+			const uint32_t *row = s_rows[wave][0], *below = s_rows[wave][1];
+			const Texel t00 = filtered(P, row, base, bx, by);
 			uint32_t c[3] = { t00.r, t00.g, t00.b };
-			int bug = 0;
-			if (P.fetch_bug) {
-				const int prev_y = (y - P.init_y_add) >> 10, next_y = (y + P.init_y_add) >> 10;
-				if (cy != 0 && by == prev_y && by != next_y) bug = 1;
-			}
-			if (P.status & VI_META_SCALE) {
-				const uint32_t xf = (uint32_t)((x >> 5) & 31), yf = (uint32_t)((y >> 5) & 31);
-				const Texel t10 = filtered(P, A, 0, bx + 1, by);
-				const Texel t01 = filtered(P, A, bug, bx, by + 1);
-				const Texel t11 = filtered(P, A, bug, bx + 1, by + 1);
-				const uint32_t v10[3] = { t10.r, t10.g, t10.b }, v01[3] = { t01.r, t01.g, t01.b };
-				const uint32_t v11[3] = { t11.r, t11.g, t11.b };
+			if (scale) {
+				const uint32_t xf = (uint32_t)((x >> 5) & 31);
+				const Texel t10 = filtered(P, row, base, bx + 1, by);
+				uint32_t r[3] = { t10.r, t10.g, t10.b };
+				if (yf) {
+					const Texel t01 = filtered(P, below, base, bx, by + 1);
+					const Texel t11 = filtered(P, below, base, bx + 1, by + 1);
+					const uint32_t v01[3] = { t01.r, t01.g, t01.b }, v11[3] = { t11.r, t11.g, t11.b };
 #pragma unroll
-				for (int i = 0; i < 3; i++) c[i] = vi_lerp(vi_lerp(c[i], v01[i], yf), vi_lerp(v10[i], v11[i], yf), xf);
+					for (int i = 0; i < 3; i++) {
+						c[i] = vi_lerp(c[i], v01[i], yf);
+						r[i] = vi_lerp(r[i], v11[i], yf);
+					}
+				}
+#pragma unroll
+				for (int i = 0; i < 3; i++) c[i] = vi_lerp(c[i], r[i], xf);
 			}
 			if (P.status & VI_GAMMA) {
 				if (P.status & VI_GAMMA_DITHER) {
@@ -471,6 +516,7 @@ __global__ __launch_bounds__(256) void k_vi_scale(const ViParams *__restrict__ p
 			result = c[0] | (c[1] << 8) | (c[2] << 16) | 0xff000000u;
 		}
 	}
+	if (px >= P.ow) return;
 	if (P.blend && (result >> 24) == 0) {
 		bool in_rect = false;
 		for (int k = 0; k < P.nrects; k++)
@@ -482,7 +528,9 @@ __global__ __launch_bounds__(256) void k_vi_scale(const ViParams *__restrict__ p
 			result = (p >> 24) ? (p & 0x00ffffffu) : 0;
 		}
 	}
-	out[(size_t)py * (size_t)P.ow + (size_t)px] = result;
+	const size_t at = (size_t)py * (size_t)P.ow + (size_t)px;
+	out[at] = result;
+	host[at] = result;
 }
 
 #define VI_CHECK(expr)                                                                                         \
@@ -515,17 +563,20 @@ hipError_t launch_domain_range(const uint8_t *rdram, const uint8_t *hidden, uint
                                uint8_t *hplanes, uint32_t rdram_size, uint32_t num_planes, uint32_t addr,
                                uint32_t num_pixels, uint32_t size_log2, hipStream_t s);
 
+// Bytes of a band of the image a waiting scanout copies to the caller's memory
+// while the next band is still being written over PCIe (one band below twice
+// this).  2560x960 pixels: 410 us in 8 bands, 530 us in one; below 1 MB a second
+// launch and wait cost what the overlap gains (1.2 MB: 88 us in one, 86 in four).
+constexpr size_t kViBandBytes = 1u << 19;
+constexpr size_t kViMaxBands = 8;
+
 int vi_scanout(ViState &s, const uint32_t *regs, const ViSource &src, const uint8_t *d_gamma, hipStream_t stream,
-               const rdp_mi_scanout_options &opts, uint32_t *out, unsigned *width, unsigned *height, bool sync)
+               const rdp_mi_scanout_options &opts, uint32_t *out, unsigned *width, unsigned *height, ViStaging *stage)
 {
 	const uint8_t *d_rdram = src.rdram, *d_hidden = src.hidden;
 	const uint32_t rdram_size = src.rdram_size;
+	const bool sync = stage != nullptr;
 	const int L = (int)src.scale_log2, SF = 1 << L;
-	if (!s.h_params) {
-		VI_CHECK(hipHostMalloc((void **)&s.h_params, sizeof(ViParams), hipHostMallocDefault));
-		VI_CHECK(hipMalloc((void **)&s.d_params, sizeof(ViParams)));
-		VI_CHECK(hipEventCreateWithFlags(&s.params_done, hipEventDisableTiming));
-	}
 	const size_t image_words = (size_t)640 * 576 << (2 * L);
 	if (s.image_words < image_words) {
 		VI_CHECK(hipStreamSynchronize(stream));
@@ -536,15 +587,12 @@ int vi_scanout(ViState &s, const uint32_t *regs, const ViSource &src, const uint
 		for (auto &img : s.d_images) VI_CHECK(hipMalloc((void **)&img, image_words * sizeof(uint32_t)));
 		s.image_words = image_words;
 	}
-	// The previous scanout's parameter upload reads the pinned block.
-	if (s.params_busy) {
-		VI_CHECK(hipEventSynchronize(s.params_done));
-		s.params_busy = false;
-	}
-	ViParams &P = *s.h_params;
+	ViParams P;
 	memset(&P, 0, sizeof(P));
 	Decoded r;
-	decode(s, regs, r, P.lines);
+	ViLine lines[kViMaxLines];
+	decode(s, regs, r, lines);
+	const bool per_line = s.per_line_ended;
 	s.per_line_flags = 0;  // clear_per_scanline_state
 	s.per_line_ended = false;
 	*width = *height = 0;
@@ -590,6 +638,9 @@ int vi_scanout(ViState &s, const uint32_t *regs, const ViSource &src, const uint
 	}
 	s.last_valid_frame_count = s.frame_count;
 	const bool degenerate = r.h_res <= 0 || r.v_res <= 0;
+	// The lines that show the registers, in native lines.
+	P.line_lo = r.v_start;
+	P.line_hi = r.v_start + r.v_res;
 
 	// video_interface.cpp:1299-1318: every coordinate scales with the factor.
 	r.h_start *= SF;
@@ -600,7 +651,7 @@ int vi_scanout(ViState &s, const uint32_t *regs, const ViSource &src, const uint
 	r.v_res *= SF;
 	r.max_x = r.max_x * SF + (SF - 1);
 	r.max_y = r.max_y * SF + (SF - 1);
-	for (ViLine &li : P.lines) {
+	for (ViLine &li : lines) {
 		li.h_start *= SF;
 		li.h_start_clamp *= SF;
 		li.h_end_clamp *= SF;
@@ -704,36 +755,54 @@ int vi_scanout(ViState &s, const uint32_t *regs, const ViSource &src, const uint
 		}
 	}
 
-	// Fetch-filter image (both layers).
-	if (!degenerate) {
-		const size_t words = (size_t)P.aw * (size_t)P.ah * 2;
-		if (words > s.filter_words) {
-			if (s.d_filter) {
-				VI_CHECK(hipStreamSynchronize(stream));
-				VI_CHECK(hipFree(s.d_filter));
-				s.d_filter = nullptr;
-			}
-			VI_CHECK(hipMalloc((void **)&s.d_filter, words * sizeof(uint32_t)));
-			s.filter_words = words;
+	// Registers latched per scanline go through memory; otherwise every shown
+	// line has the same ones, and they are kernel arguments.
+	const ViLine *d_lines = nullptr;
+	if (per_line && !degenerate) {
+		if (!s.h_lines) {
+			VI_CHECK(hipHostMalloc((void **)&s.h_lines, sizeof(lines), hipHostMallocDefault));
+			VI_CHECK(hipMalloc((void **)&s.d_lines, sizeof(lines)));
+			VI_CHECK(hipEventCreateWithFlags(&s.lines_done, hipEventDisableTiming));
 		}
-	}
-	VI_CHECK(hipMemcpyAsync(s.d_params, s.h_params, sizeof(ViParams), hipMemcpyHostToDevice, stream));
-	VI_CHECK(hipEventRecord(s.params_done, stream));
-	s.params_busy = true;
-	if (!degenerate) {
-		dim3 grid((unsigned)((P.aw + 15) / 16), (unsigned)((P.ah + 15) / 16));
-		hipLaunchKernelGGL(k_vi_filter, grid, dim3(256), 0, stream, s.d_params, d_rdram, d_hidden, s.d_filter);
-		VI_CHECK(hipGetLastError());
-	}
+		// The previous upload reads the pinned block.
+		if (s.lines_busy) {
+			VI_CHECK(hipEventSynchronize(s.lines_done));
+			s.lines_busy = false;
+		}
+		memcpy(s.h_lines, lines, sizeof(lines));
+		VI_CHECK(hipMemcpyAsync(s.d_lines, s.h_lines, sizeof(lines), hipMemcpyHostToDevice, stream));
+		VI_CHECK(hipEventRecord(s.lines_done, stream));
+		s.lines_busy = true;
+		d_lines = s.d_lines;
+	} else if (!degenerate)
+		P.line = lines[P.line_lo];
 	uint32_t *dst = s.d_images[s.cur];
 	const uint32_t *prevp = s.d_images[s.cur ^ 1];
-	{
-		dim3 grid((unsigned)((P.ow + 63) / 64), (unsigned)((P.oh + 3) / 4));
-		hipLaunchKernelGGL(k_vi_scale, grid, dim3(256), 0, stream, s.d_params, s.d_filter, d_gamma, prevp, dst);
-		VI_CHECK(hipGetLastError());
+	// The kernel writes the image into pinned host memory: the caller's buffer,
+	// or the staging block of a caller that waits, copied band by band.
+	const size_t words = (size_t)P.ow * (size_t)P.oh;
+	size_t bands = 1;
+	uint32_t *host = out;
+	if (sync) {
+		bands = std::min(std::max<size_t>(words * 4 / kViBandBytes, 1), kViMaxBands);
+		if (int err = stage->reserve(words, bands)) return err;
+		host = stage->pixels;
 	}
-	VI_CHECK(hipMemcpyAsync(out, dst, (size_t)P.ow * (size_t)P.oh * 4, hipMemcpyDeviceToHost, stream));
-	if (sync) VI_CHECK(hipStreamSynchronize(stream));
+	auto band_row = [&](size_t k) { return (int)((size_t)P.oh * k / bands); };
+	for (size_t k = 0; k < bands; k++) {
+		const int row0 = band_row(k), row1 = band_row(k + 1);
+		dim3 grid((unsigned)((P.ow + 63) / 64), (unsigned)((row1 - row0 + 3) / 4));
+		hipLaunchKernelGGL(k_vi, grid, dim3(256), 0, stream, P, d_lines, d_rdram, d_hidden, d_gamma, prevp, dst, host, row0,
+		                   row1);
+		VI_CHECK(hipGetLastError());
+		if (sync) VI_CHECK(hipEventRecord(stage->done[k], stream));
+	}
+	if (sync)
+		for (size_t k = 0; k < bands; k++) {
+			VI_CHECK(hipEventSynchronize(stage->done[k]));
+			const size_t at = (size_t)band_row(k) * (size_t)P.ow, n = (size_t)band_row(k + 1) * (size_t)P.ow - at;
+			memcpy(out + at, host + at, n * 4);
+		}
 	*width = (unsigned)P.ow;
 	*height = (unsigned)P.oh;
 	s.prev_w = (unsigned)P.ow;

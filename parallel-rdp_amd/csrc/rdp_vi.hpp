@@ -1,11 +1,13 @@
 // Video interface (VI) scanout on the device: register decode on the host,
-// then two kernels (fetch filter, then divot + scale + gamma + blend).
+// then one kernel (fetch filter, divot, scale, gamma, blend).
 // Follows parallel-rdp/video_interface.cpp:176-403, 796-998, 1126-1426 and
 // shaders/extract_vram.comp, vi_fetch.frag, vi_divot.frag, vi_scale.frag.
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <vector>
 
 #include "../../include/rdp_mi.h"
 
@@ -18,7 +20,7 @@ struct ViLine {
 	int32_t h_start, h_start_clamp, h_end_clamp, x_start, x_add, y_start, y_add, y_base;
 };
 
-// Everything the two VI kernels need for one scanout.
+// Everything the VI kernel needs for one scanout (a kernel argument).
 struct ViParams {
 	uint32_t status;
 	int32_t fb_offset, fb_width, x_off, y_off;
@@ -32,8 +34,19 @@ struct ViParams {
 	int32_t rects[3][4];
 	uint32_t rdram_mask;
 	int32_t scale_log2;  // upscaled scanout: the image is read from 4^scale_log2 sample planes
-	uint32_t pad[2];
-	ViLine lines[kViMaxLines];
+	// The registers of native lines line_lo .. line_hi - 1 when none were latched
+	// per scanline.
+	int32_t line_lo, line_hi;
+	ViLine line;
+};
+
+// Pinned host memory a waiting scanout's image passes through on its way to
+// the caller's memory (grows to the largest image), and an event per band.
+struct ViStaging {
+	uint32_t *pixels = nullptr;
+	size_t words = 0;
+	std::vector<hipEvent_t> done;
+	int reserve(size_t want, size_t bands);
 };
 
 // Where the scanout reads the frame.  scale_log2 = 0: rdram / hidden are
@@ -59,12 +72,10 @@ struct ViState {
 	uint32_t *d_images[2] = { nullptr, nullptr };  // output, ping-pong with the previous one
 	size_t image_words = 0;                         // capacity of each
 	int cur = 0;
-	uint32_t *d_filter = nullptr;                   // fetch-filter image, both layers
-	size_t filter_words = 0;
-	ViParams *h_params = nullptr;                   // pinned
-	ViParams *d_params = nullptr;
-	hipEvent_t params_done = nullptr;               // the upload of h_params has been read
-	bool params_busy = false;
+	ViLine *h_lines = nullptr;                      // pinned: registers latched per scanline
+	ViLine *d_lines = nullptr;
+	hipEvent_t lines_done = nullptr;                // the upload of h_lines has been read
+	bool lines_busy = false;
 
 	uint32_t per_line_flags = 0;
 	uint32_t h_start_latched = 0, x_scale_latched = 0;
@@ -79,17 +90,17 @@ struct ViState {
 	void release();
 };
 
-// Scans out the processor's current RDRAM through the VI into out
-// (width x height RGBA8 words, byte order R, G, B, A), queued on `stream`
-// behind the rendering.  With sync the call waits for the copy to `out`;
-// otherwise the copy is still in flight on `stream` when it returns.
-// Returns 0 or an RDP_MI_ERROR_* code.
 // RDRAM bytes [offset, offset + length) (modulo the RDRAM size) a scanout
 // with these registers fetches.
 void vi_memory_range(const ViState &vi, const uint32_t *regs, uint32_t &offset, uint32_t &length);
+// Scans out the processor's current RDRAM through the VI into out
+// (width x height RGBA8 words, byte order R, G, B, A), queued on `stream`
+// behind the rendering.  With `stage` the call waits and out is any host
+// memory; without, out is pinned and still being written when it returns.
 // With upscaling the image is up to (640 x 576) << (2 * scale_log2) words.
+// Returns 0 or an RDP_MI_ERROR_* code.
 int vi_scanout(ViState &vi, const uint32_t *regs, const ViSource &src, const uint8_t *d_gamma, hipStream_t stream,
-               const rdp_mi_scanout_options &opts, uint32_t *out, unsigned *width, unsigned *height, bool sync);
+               const rdp_mi_scanout_options &opts, uint32_t *out, unsigned *width, unsigned *height, ViStaging *stage);
 
 // Gamma table (luts.hpp:1034-1555) from its closed form, 256 + 16384 bytes.
 void vi_gamma_table(uint8_t *out);

@@ -365,7 +365,7 @@ class CommandProcessor:
         """VI scanout as a (height, width) array of RGBA8 words (R in the low byte);
         (0, 0) for a blank or invalid frame."""
         opts = options if options is not None else ScanoutOptions.default()
-        out = np.zeros(640 * 576 * self.upscaling_factor ** 2, dtype=np.uint32)
+        out = np.empty(640 * 576 * self.upscaling_factor ** 2, dtype=np.uint32)
         w = ctypes.c_uint(0)
         h = ctypes.c_uint(0)
         _check(self._lib.rdp_mi_scanout_sync_ex(self._h, ctypes.byref(opts), out.ctypes.data, ctypes.byref(w),
