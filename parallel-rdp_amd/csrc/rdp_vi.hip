@@ -565,8 +565,9 @@ hipError_t launch_domain_range(const uint8_t *rdram, const uint8_t *hidden, uint
 
 // Bytes of a band of the image a waiting scanout copies to the caller's memory
 // while the next band is still being written over PCIe (one band below twice
-// this).  2560x960 pixels: 410 us in 8 bands, 530 us in one; below 1 MB a second
-// launch and wait cost what the overlap gains (1.2 MB: 88 us in one, 86 in four).
+// this).  2560x960 pixels: 410 us in 8 bands; the kernel alone takes 220 us and
+// the copy alone 324.  Below 1 MB a further launch and wait cost what the overlap
+// gains (1.2 MB: 88 us in one band, 86 in four).
 constexpr size_t kViBandBytes = 1u << 19;
 constexpr size_t kViMaxBands = 8;
 
