@@ -7,7 +7,7 @@
 //             covered scanline (SpanSetup) and reduces the per-8-line x extent
 //             into tile-row ranges.
 //   k_tmem_gather / k_tmem_scan
-//             one lane per (block of 32 uploads, TMEM halfword) applies the
+//             one lane per (block of 8 uploads, TMEM halfword) applies the
 //             block's uploads in order; then one lane per halfword carries
 //             values across blocks, completing the TMEM snapshot after every
 //             upload.
@@ -511,13 +511,11 @@ DEV uint32_t tmem_fetch(const Mem &m, const TmemLoad &ld, bool upper, bool yuv)
 }
 
 // Stage 2 runs in two kernels so a pass's uploads are processed in parallel.
-// k_tmem_gather: one thread per (block of 32 uploads, TMEM halfword) applies
+// k_tmem_gather: one thread per (block of kTmemBlock uploads, TMEM halfword) applies
 // the block's uploads in order: from the block's first write to its halfword
 // on, every snapshot slot of the block is complete.  It records where that
 // first write is and the halfword's value after the block.  The item is
 // pass << 12 | block << 3 | 256-halfword chunk.
-constexpr int kTmemBlock = 32;
-
 __global__ __launch_bounds__(256) void k_tmem_gather(const PassDesc *__restrict__ passes,
                                                      const uint32_t *__restrict__ items)
 {
@@ -559,8 +557,11 @@ __global__ __launch_bounds__(256) void k_tmem_scan(const PassDesc *__restrict__ 
 	P.tmem_instances[g] = (uint16_t)carry;
 	const int n = (int)P.num_uploads;
 	const int blocks = (n + kTmemBlock - 1) / kTmemBlock;
+	uint32_t next = blocks ? P.tmem_blocks[g] : 0;
 	for (int b = 0; b < blocks; b++) {
-		const uint32_t info = P.tmem_blocks[b * 2048 + g];
+		const uint32_t info = next;
+		// The next block's record, fetched before this block's stores.
+		if (b + 1 < blocks) next = P.tmem_blocks[(b + 1) * 2048 + g];
 		const int i0 = b * kTmemBlock;
 		const int count = imin(kTmemBlock, n - i0);
 		const int first = (int)(info >> 16);

@@ -417,7 +417,7 @@ static ScratchLayout scratch_layout(const HostPass &hp)
 	l.tilerows = align_up((size_t)hp.num_tilerows * 4, 256);
 	l.bins = align_up((size_t)tx * ty * groups * 8, 256);
 	l.tmem = align_up((hp.uploads.size() + 1) * 4096, 256);
-	l.tmem_blocks = align_up(std::max<size_t>((hp.uploads.size() + 31) / 32, 1) * 2048 * 4, 256);
+	l.tmem_blocks = align_up(std::max<size_t>(tmem_blocks(hp.uploads.size()), 1) * 2048 * 4, 256);
 	l.psetups = align_up(hp.prims.size() * sizeof(PrimSetup), 256);
 	l.tilerow_prim = align_up((size_t)hp.num_tilerows * 2, 256);
 	l.total = l.setups + l.spans + l.tilerows + l.bins + l.tmem + l.tmem_blocks + l.psetups + l.tilerow_prim;
@@ -757,7 +757,7 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 			// TMEM snapshots.
 			if (!up) {
 				L.n_tmem += 8;
-				L.n_tmem_gather += 8 * (uint32_t)((hp.uploads.size() + 31) / 32);
+				L.n_tmem_gather += 8 * tmem_blocks(hp.uploads.size());
 			}
 			if (hp.domain_pre) L.n_dom_pre += domain_blocks(hp);
 			if (hp.domain_post) L.n_dom_post += domain_blocks(hp);
@@ -985,7 +985,7 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 			for (uint32_t b = 0; b < (D.num_tilerows + 7) / 8; b++) it_setup[L.n_setup + nsp++] = (pidx << 17) | b;
 			if (!hp.scale_log2) {
 				for (uint32_t k = 0; k < 8; k++) it_tmem[L.n_tmem_gather + nt++] = (pidx << 12) | k;
-				for (uint32_t b = 0; b < (uint32_t)(hp.uploads.size() + 31) / 32; b++)
+				for (uint32_t b = 0; b < tmem_blocks(hp.uploads.size()); b++)
 					for (uint32_t k = 0; k < 8; k++) it_tmem[ntg++] = (pidx << 12) | (b << 3) | k;
 			}
 			if (D.num_prims) {
