@@ -39,6 +39,25 @@ inline void pass_write_ranges(const HostPass &hp, std::vector<ByteRange> &out)
 	}
 }
 
+// The same for native RDRAM when the pass may be an upscaled one: its raster
+// writes the sample planes only, and with a resolve also its native region.
+inline void native_write_ranges(const HostPass &hp, std::vector<ByteRange> &out)
+{
+	if (!hp.scale_log2) {
+		pass_write_ranges(hp, out);
+		return;
+	}
+	if (!hp.ssaa_resolve || hp.prims.empty()) return;
+	const uint64_t px = (uint64_t)(hp.fb_width >> hp.scale_log2) * hp.domain_height;
+	const uint32_t log2 = hp.fb_fmt == FB_RGBA8888 ? 2 : (hp.fb_fmt == FB_RGBA5551 || hp.fb_fmt == FB_IA88) ? 1 : 0;
+	const uint64_t base = (hp.fb_addr >> log2) << log2;
+	out.push_back({ base & ~3ull, (base + (px << log2) + 3) & ~3ull });
+	if (hp.depth_addr != hp.fb_addr) {
+		const uint64_t dep = hp.depth_addr & ~1u;
+		out.push_back({ dep & ~3ull, (dep + 2 * px + 3) & ~3ull });
+	}
+}
+
 // A bound on the RDRAM bytes a TMEM upload reads: rows 0 .. height-1 of the
 // source image (vram_width texels apart, at most 4 bytes each) and, for
 // TLUT loads, vram_effective_width entries from vram_addr.  False when the

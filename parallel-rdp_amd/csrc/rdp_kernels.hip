@@ -2,15 +2,14 @@
 //
 // Four stages per render pass (any number of passes, from any number of
 // streams, per launch; every block finds its pass through a work item):
-//   k_setup   one wave64 per primitive: decodes the raw command words with the
-//             pass draw state, writes PrimSetup, walks the edges for every
-//             covered scanline (SpanSetup) and reduces the per-8-line x extent
-//             into tile-row ranges.
-//   k_tmem_gather / k_tmem_scan
-//             one lane per (block of 8 uploads, TMEM halfword) applies the
-//             block's uploads in order; then one lane per halfword carries
-//             values across blocks, completing the TMEM snapshot after every
-//             upload.
+//   k_prep    one lane per primitive decodes the raw command words with the
+//             pass draw state and writes RasterPrim and PrimSetup; in blocks of
+//             their own, one lane per (block of 8 uploads, TMEM halfword) applies
+//             the block's uploads in order.
+//   k_rows    one lane per scanline walks a primitive's edges (SpanSetup) and
+//             reduces the per-8-line x extent into tile-row ranges; in blocks of
+//             their own, one lane per TMEM halfword carries values across the
+//             blocks of uploads, completing the TMEM snapshot after every upload.
 //   k_bin     one wave64 per (tile row, group of 64 primitives): a ballot per
 //             tile column produces the ordered 64-bit primitive masks.
 //   k_raster  one wave64 per 8x8 screen tile: colour/depth/coverage of the 64
@@ -371,17 +370,16 @@ DEV void compute_span(const PrimSetup &s, Scissor sc, int y, SpanSetup &out, int
 	out.lodlength = (int16_t)(flip ? (out.end_x - out.base_x) : (out.base_x - out.start_x));
 }
 
-// Setup runs in two launches.  k_setup: one lane per primitive decodes its
-// command words and draw state, writes the RasterPrim record and the decoded
-// PrimSetup, and marks which primitive owns each of its tile-row entries.
-// k_span: one wave per 8 tile-row entries, one lane per span row: the rows
-// of small triangles pack densely into waves and a tall triangle spreads over
-// many waves.
-__global__ __launch_bounds__(64) void k_setup(const PassDesc *__restrict__ passes, const uint32_t *__restrict__ items)
+// Setup runs in two launches.  k_prep's setup items: one lane per primitive
+// decodes its command words and draw state, writes the RasterPrim record and the
+// decoded PrimSetup, and marks which primitive owns each of its tile-row entries.
+// k_rows' span items: one wave per 8 tile-row entries, one lane per span row: the
+// rows of small triangles pack densely into waves and a tall triangle spreads
+// over many waves.
+DEV void setup_item(const PassDesc *__restrict__ passes, uint32_t item, uint32_t lane)
 {
-	const uint32_t item = items[blockIdx.x];
 	const PassDesc &P = passes[item >> 7];
-	const uint32_t prim = (item & 0x7f) * 64 + threadIdx.x;
+	const uint32_t prim = (item & 0x7f) * 64 + lane;
 	if (prim >= P.num_prims) return;
 
 	const PrimRecord &rec = P.prims[prim];
@@ -437,7 +435,7 @@ __global__ __launch_bounds__(64) void k_setup(const PassDesc *__restrict__ passe
 	P.rprims[prim] = r;
 	P.psetups[prim] = s;
 
-	// Spans cover rows ylo .. yhi + 1 and k_span covers the tile rows
+	// Spans cover rows ylo .. yhi + 1 and the span items cover the tile rows
 	// ylo / 8 .. yhi / 8; row yhi + 1 lies beyond them when it starts a new
 	// tile row, and is done here.
 	const int rows = (s.yhi >> 3) - (s.ylo >> 3) + 1;
@@ -449,15 +447,9 @@ __global__ __launch_bounds__(64) void k_setup(const PassDesc *__restrict__ passe
 	}
 }
 
-#ifndef RDP_SPAN_WAVES
-#define RDP_SPAN_WAVES 6
-#endif
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(RDP_SPAN_WAVES)))
-void k_span(const PassDesc *__restrict__ passes, const uint32_t *__restrict__ items)
+DEV void span_item(const PassDesc *__restrict__ passes, uint32_t item, int lane)
 {
-	const uint32_t item = items[blockIdx.x];
 	const PassDesc &P = passes[item >> 17];
-	const int lane = threadIdx.x;
 	const uint32_t e = (item & 0x1ffff) * 8 + (uint32_t)(lane >> 3);
 	const bool live = e < P.num_tilerows;
 	int tlo = 0x7fffffff, thi = -1;
@@ -510,18 +502,16 @@ DEV uint32_t tmem_fetch(const Mem &m, const TmemLoad &ld, bool upper, bool yuv)
 	return word;
 }
 
-// Stage 2 runs in two kernels so a pass's uploads are processed in parallel.
-// k_tmem_gather: one thread per (block of kTmemBlock uploads, TMEM halfword) applies
+// Stage 2 runs in two steps so a pass's uploads are processed in parallel.
+// Gather: one thread per (block of kTmemBlock uploads, TMEM halfword) applies
 // the block's uploads in order: from the block's first write to its halfword
-// on, every snapshot slot of the block is complete.  It records where that
-// first write is and the halfword's value after the block.  The item is
+// on, every snapshot slot of the block is complete.  It records which upload
+// makes that first write (kTmemBlock: none).  The item is
 // pass << 12 | block << 3 | 256-halfword chunk.
-__global__ __launch_bounds__(256) void k_tmem_gather(const PassDesc *__restrict__ passes,
-                                                     const uint32_t *__restrict__ items)
+DEV void gather_item(const PassDesc *__restrict__ passes, uint32_t item, uint32_t thread)
 {
-	const uint32_t item = items[blockIdx.x];
 	const PassDesc &P = passes[item >> 12];
-	const int g = (int)((item & 7) * 256 + threadIdx.x);  // 0..2047
+	const int g = (int)((item & 7) * 256 + thread);  // 0..2047
 	const int block = (int)((item >> 3) & 0x1ff);
 	const int i0 = block * kTmemBlock;
 	const Mem m{ gptr(P.rdram), gptr(P.hidden), P.rdram_mask };
@@ -540,36 +530,81 @@ __global__ __launch_bounds__(256) void k_tmem_gather(const PassDesc *__restrict_
 		}
 		if (first != kTmemBlock) P.tmem_instances[(i + 1) * 2048 + g] = (uint16_t)cur;
 	}
-	P.tmem_blocks[block * 2048 + g] = ((uint32_t)first << 16) | cur;
+	P.tmem_first[block * 2048 + g] = (uint8_t)first;
 }
 
-// k_tmem_scan: one thread per TMEM halfword walks the blocks in order,
-// filling each block's slots before its first write with the value carried
-// from the blocks before (the last writer wins), then writes the final TMEM
-// back to the stream.  The item is pass << 12 | 256-halfword chunk.
-__global__ __launch_bounds__(256) void k_tmem_scan(const PassDesc *__restrict__ passes,
-                                                   const uint32_t *__restrict__ items)
+// Scan: one thread per TMEM halfword walks the blocks in order, filling each
+// block's slots before its first write with the value carried from the blocks
+// before (the last writer wins; the value after a block with a write is its
+// last slot), then goes on to the stream's next pass of the launch, and writes
+// the final TMEM back to the stream.  The item is
+// pass << 12 | 256-halfword chunk.
+DEV void scan_item(const PassDesc *__restrict__ passes, uint32_t item, uint32_t thread)
 {
-	const uint32_t item = items[blockIdx.x];
-	const PassDesc &P = passes[item >> 12];
-	const int g = (int)((item & 7) * 256 + threadIdx.x);
-	uint32_t carry = P.tmem[g];
-	P.tmem_instances[g] = (uint16_t)carry;
-	const int n = (int)P.num_uploads;
-	const int blocks = (n + kTmemBlock - 1) / kTmemBlock;
-	uint32_t next = blocks ? P.tmem_blocks[g] : 0;
-	for (int b = 0; b < blocks; b++) {
-		const uint32_t info = next;
+	const PassDesc *P = &passes[item >> 12];
+	const int g = (int)((item & 7) * 256 + thread);
+	uint32_t carry = P->tmem[g];
+	for (;;) {
+		uint16_t *slots = P->tmem_instances;
+		slots[g] = (uint16_t)carry;
+		const int n = (int)P->num_uploads;
+		const int blocks = (n + kTmemBlock - 1) / kTmemBlock;
+		int next_first = 0;
+		uint32_t next_value = 0;
 		// The next block's record, fetched before this block's stores.
-		if (b + 1 < blocks) next = P.tmem_blocks[(b + 1) * 2048 + g];
-		const int i0 = b * kTmemBlock;
-		const int count = imin(kTmemBlock, n - i0);
-		const int first = (int)(info >> 16);
-		const int gap = imin(first, count);
-		for (int k = 0; k < gap; k++) P.tmem_instances[(i0 + k + 1) * 2048 + g] = (uint16_t)carry;
-		if (first < count) carry = info & 0xffff;
+		auto fetch = [&](int b) {
+			if (b >= blocks) return;
+			next_first = P->tmem_first[b * 2048 + g];
+			next_value = slots[imin((b + 1) * kTmemBlock, n) * 2048 + g];
+		};
+		fetch(0);
+		for (int b = 0; b < blocks; b++) {
+			const int first = next_first;
+			const uint32_t value = next_value;
+			fetch(b + 1);
+			const int i0 = b * kTmemBlock;
+			const int count = imin(kTmemBlock, n - i0);
+			const int gap = imin(first, count);
+			for (int k = 0; k < gap; k++) slots[(i0 + k + 1) * 2048 + g] = (uint16_t)carry;
+			if (first < count) carry = value;
+		}
+		const uint32_t step = P->tmem_next;
+		if (!step) break;
+		P += step;
 	}
-	P.tmem[g] = (uint16_t)carry;
+	P->tmem[g] = (uint16_t)carry;
+}
+
+// Setup and TMEM replay share two launches: neither needs the other, and one
+// frame fills the GPU with neither.  k_prep: blocks of 256 TMEM halfwords (the
+// gather, the longer chain, first), then four waves of 64 primitives each.
+__global__ __launch_bounds__(256) void k_prep(const PassDesc *__restrict__ passes, const uint32_t *__restrict__ gather_items,
+                                              uint32_t n_gather, const uint32_t *__restrict__ setup_items,
+                                              uint32_t n_setup)
+{
+	if (blockIdx.x < n_gather) {
+		gather_item(passes, gather_items[blockIdx.x], threadIdx.x);
+		return;
+	}
+	const uint32_t k = (blockIdx.x - n_gather) * 4 + uniform_u32(threadIdx.x >> 6);
+	if (k < n_setup) setup_item(passes, setup_items[k], threadIdx.x & 63);
+}
+
+// k_rows: the TMEM scan of 256 halfwords per block, then four waves of 8
+// tile-row entries each.
+#ifndef RDP_SPAN_WAVES
+#define RDP_SPAN_WAVES 6
+#endif
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RDP_SPAN_WAVES)))
+void k_rows(const PassDesc *__restrict__ passes, const uint32_t *__restrict__ scan_items, uint32_t n_scan,
+            const uint32_t *__restrict__ span_items, uint32_t n_span)
+{
+	if (blockIdx.x < n_scan) {
+		scan_item(passes, scan_items[blockIdx.x], threadIdx.x);
+		return;
+	}
+	const uint32_t k = (blockIdx.x - n_scan) * 4 + uniform_u32(threadIdx.x >> 6);
+	if (k < n_span) span_item(passes, span_items[k], (int)(threadIdx.x & 63));
 }
 
 // ==========================================================================
@@ -2551,19 +2586,37 @@ void k_raster_round(const PassDesc *__restrict__ passes, const uint32_t *__restr
 // ==========================================================================
 // Launchers (host side).
 // ==========================================================================
-hipError_t launch_setup(const PassDesc *passes, const uint32_t *items, uint32_t n, const uint32_t *span_items,
-                        uint32_t n_span, hipStream_t s)
+// Packed inputs from pinned host memory, 16 bytes per lane and step.  A kernel
+// reads over PCIe at the copy engine's rate (715 KB: 14 us) and the launches
+// behind it follow in stream order, without the engine's hand-over (64 KB and a
+// launch: 14.5 against 20 us; 600 KB: 25 against 30; 10 MB: 190 either way).
+__global__ __launch_bounds__(256) void k_upload(const uint4 *__restrict__ src, uint4 *__restrict__ dst, uint32_t n)
 {
-	if (n) hipLaunchKernelGGL(k_setup, dim3(n), dim3(64), 0, s, passes, items);
-	if (n_span) hipLaunchKernelGGL(k_span, dim3(n_span), dim3(64), 0, s, passes, span_items);
+	for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
+}
+
+hipError_t launch_upload(const void *pinned, void *dst, size_t bytes, hipStream_t s)
+{
+	const uint32_t n = (uint32_t)(bytes / 16);
+	if (!n) return hipSuccess;
+	hipLaunchKernelGGL(k_upload, dim3(n < 256 * 256 ? (n + 255) / 256 : 256), dim3(256), 0, s, (const uint4 *)pinned,
+	                   (uint4 *)dst, n);
 	return hipGetLastError();
 }
 
-hipError_t launch_tmem(const PassDesc *passes, const uint32_t *gather_items, uint32_t n_gather,
-                       const uint32_t *scan_items, uint32_t n_scan, hipStream_t s)
+// Setup (n_setup items of 64 primitives, then n_span of 8 tile-row entries)
+// and TMEM replay (n_gather and n_scan items of 256 halfwords); either may be
+// absent.
+hipError_t launch_prep(const PassDesc *passes, const uint32_t *setup_items, uint32_t n_setup, const uint32_t *span_items,
+                       uint32_t n_span, const uint32_t *gather_items, uint32_t n_gather, const uint32_t *scan_items,
+                       uint32_t n_scan, hipStream_t s)
 {
-	if (n_gather) hipLaunchKernelGGL(k_tmem_gather, dim3(n_gather), dim3(256), 0, s, passes, gather_items);
-	if (n_scan) hipLaunchKernelGGL(k_tmem_scan, dim3(n_scan), dim3(256), 0, s, passes, scan_items);
+	if (n_setup || n_gather)
+		hipLaunchKernelGGL(k_prep, dim3(n_gather + (n_setup + 3) / 4), dim3(256), 0, s, passes, gather_items, n_gather,
+		                   setup_items, n_setup);
+	if (n_span || n_scan)
+		hipLaunchKernelGGL(k_rows, dim3(n_scan + (n_span + 3) / 4), dim3(256), 0, s, passes, scan_items, n_scan, span_items,
+		                   n_span);
 	return hipGetLastError();
 }
 

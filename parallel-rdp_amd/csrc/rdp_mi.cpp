@@ -7,8 +7,9 @@
 //
 // Submission groups pending render passes into rounds: round r holds the
 // r-th pending pass of every participating processor.  All inputs of all
-// rounds go to the device in one copy; each round is then four launches
-// (setup, TMEM, bin, raster) whose blocks cover every pass of the round.
+// rounds go to the device in one copy.  Setup, TMEM replay and binning then
+// cover a group of rounds (small ones) or one round (many passes) per launch,
+// the raster one round; the blocks of a launch cover every pass of it.
 #include <hip/hip_runtime.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -39,8 +40,9 @@
 
 namespace rdp_mi {
 
-hipError_t launch_setup(const PassDesc *, const uint32_t *, uint32_t, const uint32_t *, uint32_t, hipStream_t);
-hipError_t launch_tmem(const PassDesc *, const uint32_t *, uint32_t, const uint32_t *, uint32_t, hipStream_t);
+hipError_t launch_upload(const void *pinned, void *dst, size_t bytes, hipStream_t s);
+hipError_t launch_prep(const PassDesc *, const uint32_t *setup, uint32_t, const uint32_t *span, uint32_t,
+                       const uint32_t *gather, uint32_t, const uint32_t *scan, uint32_t, hipStream_t);
 hipError_t launch_bin(const PassDesc *, const uint32_t *, uint32_t, hipStream_t);
 hipError_t launch_raster(uint32_t cls, const PassDesc *, const uint32_t *, uint32_t, int32_t, bool, hipStream_t);
 hipError_t launch_raster_fill(const PassDesc *, const uint32_t *, uint32_t, int32_t, hipStream_t);
@@ -397,7 +399,7 @@ struct PassRef {
 
 // Byte sizes of the per-pass device scratch.
 struct ScratchLayout {
-	size_t setups, spans, tilerows, bins, tmem, tmem_blocks, psetups, tilerow_prim, total;
+	size_t setups, spans, tilerows, bins, tmem, tmem_first, psetups, tilerow_prim, total;
 };
 
 // Bin groups of a pass: one per 64 primitives, padded to a multiple of 8 so
@@ -417,23 +419,30 @@ static ScratchLayout scratch_layout(const HostPass &hp)
 	l.tilerows = align_up((size_t)hp.num_tilerows * 4, 256);
 	l.bins = align_up((size_t)tx * ty * groups * 8, 256);
 	l.tmem = align_up((hp.uploads.size() + 1) * 4096, 256);
-	l.tmem_blocks = align_up(std::max<size_t>(tmem_blocks(hp.uploads.size()), 1) * 2048 * 4, 256);
+	l.tmem_first = (size_t)std::max(tmem_blocks(hp.uploads.size()), 1u) * 2048;
 	l.psetups = align_up(hp.prims.size() * sizeof(PrimSetup), 256);
 	l.tilerow_prim = align_up((size_t)hp.num_tilerows * 2, 256);
-	l.total = l.setups + l.spans + l.tilerows + l.bins + l.tmem + l.tmem_blocks + l.psetups + l.tilerow_prim;
+	l.total = l.setups + l.spans + l.tilerows + l.bins + l.tmem + l.tmem_first + l.psetups + l.tilerow_prim;
 	return l;
 }
 
-// One round: the four stage launches covering every pass of the round (the
-// raster stage as one launch per occupancy class present).
+// One round: the stage launches covering every pass of the round (the raster
+// stage as one launch per occupancy class present).
 struct Launch {
-	const PassDesc *descs;
-	const uint32_t *items[4];  // setup, TMEM gather, bin, raster
-	uint32_t n[4];
-	const uint32_t *tmem_scan_items;
-	uint32_t tmem_scan_n;
-	const uint32_t *span_items;  // second setup launch: one item per 8 tile-row entries
-	uint32_t span_n;
+	const PassDesc *descs;  // the round's passes: raster, domain and resolve items count from here
+	// Setup, span, bin and TMEM items count from the first pass of the round's
+	// group.  A group is one round with its own launches (prep_ahead), or
+	// consecutive small rounds whose launches are shared: at the group's first
+	// round (group_rounds != 0) the lists of the whole group are contiguous,
+	// group_* items long.
+	const PassDesc *prep_descs;
+	const uint32_t *setup_items, *span_items, *bin_items, *gather_items, *scan_items;
+	uint32_t setup_n, span_n, bin_n, gather_n, scan_n;
+	uint32_t group_rounds, group_setup, group_span, group_bin, group_gather, group_scan;
+	// The group's TMEM replay is part of its shared launches (no upload of the
+	// group reads what a raster of the group may write); otherwise each round
+	// replays its own before its raster.
+	bool group_tmem;
 	// The setup, span and bin items of passes above occupancy class 0 come
 	// first in their lists: run ahead on their own, they let the heavier
 	// classes' raster start while the light passes are still being set up.
@@ -455,7 +464,7 @@ struct Launch {
 	uint32_t up_fill_n;
 	const uint32_t *resolve_items;  // the round's upscaled passes with a resolve, after their raster
 	uint32_t resolve_n;
-	bool prep_ahead;  // every round has its own scratch: setup/binning may run ahead
+	bool prep_ahead;  // a round of many passes is present: every round has its own scratch, setup/binning run ahead
 	bool tmem_early;  // no upload reads what the previous round's raster writes
 	uint64_t raster_bytes;  // algorithmic framebuffer bytes read + written by k_raster
 	uint64_t class_bytes[kRasterClasses], fill_bytes;  // the same per raster launch
@@ -470,21 +479,20 @@ struct Launch {
 // (profiling): begin and end of k_raster_fill, then of each class launch.
 constexpr size_t kRasterEventsPerRound = 2 * (1 + kRasterClasses);
 
-// Whether round r's TMEM replay may start before round r-1's raster: no
-// upload of a pass reads RDRAM that the same processor's pass in round r-1
+// Whether round r's TMEM replay may start before round q's raster: no
+// upload of a pass reads RDRAM that the same processor's pass in round q
 // can write.
-static bool tmem_may_start_early(const std::vector<std::vector<PassRef>> &rounds, size_t r)
+static bool tmem_may_start_before(const std::vector<std::vector<PassRef>> &rounds, size_t r, size_t q)
 {
-	if (r == 0) return false;
 	std::vector<ByteRange> writes;
 	for (const PassRef &cur : rounds[r]) {
 		if (cur.pass->uploads.empty()) continue;
 		const HostPass *prev = nullptr;
-		for (const PassRef &p : rounds[r - 1])
+		for (const PassRef &p : rounds[q])
 			if (p.proc == cur.proc) prev = p.pass;
 		if (!prev) continue;
 		writes.clear();
-		pass_write_ranges(*prev, writes);
+		native_write_ranges(*prev, writes);
 		for (const UploadInfo &u : cur.pass->uploads) {
 			ByteRange rd;
 			if (!upload_read_range(u, rd)) return false;
@@ -493,6 +501,19 @@ static bool tmem_may_start_early(const std::vector<std::vector<PassRef>> &rounds
 		}
 	}
 	return true;
+}
+
+// Whether anything of a native pass reads TMEM snapshots: uploads (the snapshots
+// after them, and the stream's TMEM at the end), a state that samples or, with
+// super-sampled readback (where the native pass keeps its uploads only), the
+// upscaled copy that follows it.
+static bool needs_tmem(const PassRef &pr)
+{
+	const HostPass &hp = *pr.pass;
+	if (!hp.uploads.empty() || pr.proc->ssaa) return true;
+	for (const DrawState &d : hp.states)
+		if (d.ras_flags & (RAS_USES_TEXEL0 | RAS_USES_TEXEL1 | RAS_USES_PIPELINED_TEXEL1 | RAS_COPY)) return true;
+	return false;
 }
 
 // Blocks of 256 elements of a native pass's domain update: the framebuffer
@@ -550,18 +571,20 @@ static uint64_t framebuffer_bytes(const HostPass &hp)
 //     so the light launch fills the GPU while the heavy one's long per-tile
 //     chains finish;
 //   - the main stream joins everything back before the next round's TMEM.
-// Rounds of a few passes (the plain path, small serving batches) stay in
-// series, where the events cost more than they hide; stage timing
-// (stage_events) needs the stages in series too.
+// Submissions whose rounds all have few passes (the plain path, small serving
+// batches) stay in series, where the events cost more than they hide, with one
+// set of setup, TMEM and bin launches per group of rounds: a frame of a clear and
+// a textured pass is 6 launches instead of 13, each 4.7 us of GPU time and
+// 2.5 us of host time at least.  Stage timing (stage_events) needs the stages in
+// series too.
 constexpr uint32_t kOverlapMinPasses = 8;
 
 static int execute_launches(const std::vector<Launch> &launches, Lane &lane, const LaunchConfig &cfg,
                             hipEvent_t *stage_events = nullptr, hipEvent_t *raster_events = nullptr)
 {
 	hipStream_t s = lane.stream, side = lane.side, prep = lane.prep;
-	const bool overlap = !stage_events && side && prep;
-	const bool ahead = overlap && !launches.empty() && launches[0].prep_ahead;
-	if (overlap)
+	const bool ahead = !stage_events && side && prep && !launches.empty() && launches[0].prep_ahead;
+	if (ahead)
 		if (int err = lane.ensure_round_events(launches.size())) return err;
 	if (ahead) {
 		HIP_CHECK(hipEventRecord(lane.start, s));
@@ -569,20 +592,23 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 		for (size_t r = 0; r < launches.size(); r++) {
 			const Launch &L = launches[r];
 			// The heavier classes' passes first (prep_heavy), then the rest.
-			HIP_CHECK(launch_setup(L.descs, L.items[0], L.setup_hi, L.span_items, L.span_hi, prep));
-			HIP_CHECK(launch_bin(L.descs, L.items[2], L.bin_hi, prep));
+			HIP_CHECK(launch_prep(L.prep_descs, L.setup_items, L.setup_hi, L.span_items, L.span_hi, nullptr, 0, nullptr, 0, prep));
+			HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.bin_hi, prep));
 			HIP_CHECK(hipEventRecord(lane.events[r].prep_heavy, prep));
-			HIP_CHECK(launch_setup(L.descs, L.items[0] + L.setup_hi, L.n[0] - L.setup_hi, L.span_items + L.span_hi,
-			                       L.span_n - L.span_hi, prep));
-			HIP_CHECK(launch_bin(L.descs, L.items[2] + L.bin_hi, L.n[2] - L.bin_hi, prep));
+			HIP_CHECK(launch_prep(L.prep_descs, L.setup_items + L.setup_hi, L.setup_n - L.setup_hi, L.span_items + L.span_hi,
+			                      L.span_n - L.span_hi, nullptr, 0, nullptr, 0, prep));
+			HIP_CHECK(launch_bin(L.prep_descs, L.bin_items + L.bin_hi, L.bin_n - L.bin_hi, prep));
 			HIP_CHECK(hipEventRecord(lane.events[r].prep_done, prep));
 		}
 	}
 	bool prev_tmem_forked = false;
 	for (size_t r = 0; r < launches.size(); r++) {
 		const Launch &L = launches[r];
-		const bool big = overlap && L.passes >= kOverlapMinPasses;
-		const bool fork_tmem = big && L.tmem_scan_n;
+		const bool big = ahead && L.passes >= kOverlapMinPasses;
+		const bool fork_tmem = big && L.scan_n;
+		auto launch_tmem = [&](hipStream_t st) {
+			return launch_prep(L.prep_descs, nullptr, 0, nullptr, 0, L.gather_items, L.gather_n, L.scan_items, L.scan_n, st);
+		};
 		// Raster launches after the class floor: the merged light launch and
 		// the heavier classes.
 		const uint32_t lo = std::min(cfg.min_class, kRasterClasses - 1);
@@ -595,7 +621,7 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 		const bool persist = cfg.persistent && !raster_events && L.raster_n[kRasterClasses - 1] == 0 &&
 		                     L.raster_n[0] + L.raster_n[1] + L.fill_n > 0;
 		const bool fork_raster = big && merged && heavy && !persist;
-		const RoundEvents E = overlap ? lane.events[r] : RoundEvents();
+		const RoundEvents E = ahead ? lane.events[r] : RoundEvents();
 
 		const bool early = fork_tmem && L.tmem_early && r > 0;
 		if (fork_tmem) {
@@ -611,22 +637,34 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 			hipEvent_t after = E.fork;
 			if (early) after = (r == 1 && ahead && prev_tmem_forked) ? lane.start : lane.events[r - 1].pre_raster;
 			HIP_CHECK(hipStreamWaitEvent(side, after, 0));
-			HIP_CHECK(launch_tmem(L.descs, L.items[1], L.n[1], L.tmem_scan_items, L.tmem_scan_n, side));
+			HIP_CHECK(launch_tmem(side));
 			HIP_CHECK(hipEventRecord(E.tmem_done, side));
 		}
-		prev_tmem_forked = fork_tmem || !L.tmem_scan_n;
+		prev_tmem_forked = fork_tmem || !L.scan_n;
 		if (ahead) {
-			if (!fork_tmem) HIP_CHECK(launch_tmem(L.descs, L.items[1], L.n[1], L.tmem_scan_items, L.tmem_scan_n, s));
+			if (!fork_tmem) HIP_CHECK(launch_tmem(s));
 			HIP_CHECK(hipStreamWaitEvent(s, E.prep_done, 0));
+			HIP_CHECK(hipEventRecord(E.pre_raster, s));
+		} else if (stage_events) {
+			if (L.group_rounds)
+				HIP_CHECK(launch_prep(L.prep_descs, L.setup_items, L.group_setup, L.span_items, L.group_span, nullptr, 0, nullptr, 0, s));
+			HIP_CHECK(hipEventRecord(stage_events[r * 4 + 0], s));
+			if (!L.group_tmem)
+				HIP_CHECK(launch_tmem(s));
+			else if (L.group_rounds)
+				HIP_CHECK(launch_prep(L.prep_descs, nullptr, 0, nullptr, 0, L.gather_items, L.group_gather, L.scan_items, L.group_scan, s));
+			HIP_CHECK(hipEventRecord(stage_events[r * 4 + 1], s));
+			if (L.group_rounds) HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.group_bin, s));
+			HIP_CHECK(hipEventRecord(stage_events[r * 4 + 2], s));
 		} else {
-			HIP_CHECK(launch_setup(L.descs, L.items[0], L.n[0], L.span_items, L.span_n, s));
-			if (stage_events) HIP_CHECK(hipEventRecord(stage_events[r * 4 + 0], s));
-			if (!fork_tmem) HIP_CHECK(launch_tmem(L.descs, L.items[1], L.n[1], L.tmem_scan_items, L.tmem_scan_n, s));
-			if (stage_events) HIP_CHECK(hipEventRecord(stage_events[r * 4 + 1], s));
-			HIP_CHECK(launch_bin(L.descs, L.items[2], L.n[2], s));
-			if (stage_events) HIP_CHECK(hipEventRecord(stage_events[r * 4 + 2], s));
+			if (L.group_rounds) {
+				const uint32_t gather = L.group_tmem ? L.group_gather : 0, scan = L.group_tmem ? L.group_scan : 0;
+				HIP_CHECK(launch_prep(L.prep_descs, L.setup_items, L.group_setup, L.span_items, L.group_span, L.gather_items, gather,
+				                      L.scan_items, scan, s));
+				HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.group_bin, s));
+			}
+			if (!L.group_tmem) HIP_CHECK(launch_tmem(s));
 		}
-		if (overlap) HIP_CHECK(hipEventRecord(E.pre_raster, s));
 		// The domain's pre update reads native RDRAM before this round's
 		// raster writes it (submit_render_pass, rdp_renderer.cpp:2240-2246).
 		HIP_CHECK(launch_domain(L.descs, L.domain_pre_items, L.domain_pre_n, false, s));
@@ -690,6 +728,12 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 	return 0;
 }
 
+// Limits of a group of rounds that share setup launches: scratch (a frame of
+// 8192 small triangles takes about 25 MB) and the 15 bits of a work item's pass
+// index.
+constexpr size_t kGroupScratchBytes = 64u << 20;
+constexpr uint32_t kGroupMaxPasses = 1u << 12;
+
 // Pack the inputs of all rounds into `input` (one async copy on the context
 // stream) and describe the launches.  Caller holds the context lock.
 static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &rounds, DeviceBuffer &input,
@@ -703,15 +747,22 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 		c.staging_busy = false;
 	}
 
-	// Input layout: per round [PassDesc x n][items: setup|tmem|bin|raster], then per pass data.
+	// Input layout: per round [items: raster|domain|upscaled] and per pass data, then
+	// the descriptors and the setup, span, bin and TMEM items of all rounds.
 	struct RoundLayout {
-		size_t descs, items_setup, items_tmem, items_bin, items_raster, items_domain, items_up;
-		uint32_t n_setup, n_span, n_tmem, n_tmem_gather, n_bin, n_raster, n_fill, n_quad;
+		size_t items_raster, items_domain, items_up;
+		uint32_t n_setup, n_span, n_scan, n_gather, n_bin, n_raster, n_fill, n_quad;
+		uint32_t first_pass, group;  // index of the round's first pass; its group
 		uint32_t n_raster_class[kRasterClasses], n_quad_class[kRasterClasses];
 		uint32_t n_dom_pre, n_dom_post, n_up, n_up_class[kRasterClasses], n_up_fill, n_resolve;
-		size_t scratch;
 	};
 	std::vector<RoundLayout> rl(rounds.size());
+	// Rounds whose setup, TMEM and bin launches are shared.
+	struct Group {
+		size_t first, rounds;
+		bool tmem;
+	};
+	std::vector<Group> groups;
 	struct PassInputs {
 		size_t words, states, prims, uploads;
 		ScratchLayout sl;
@@ -722,27 +773,46 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 
 	// Submissions with a round of many passes run every round's setup and
 	// binning ahead on the lane's prep stream (execute_launches), so each
-	// round keeps its own scratch region; otherwise rounds run in series and
-	// share one region.
-	// An upscaled pass reads the TMEM snapshots its native pass (the round
-	// before) left in that round's scratch, so upscaled submissions keep
-	// every round's scratch too.
+	// round keeps its own scratch region and is a group of its own.  Otherwise
+	// rounds run in series: consecutive rounds form a group while their scratch
+	// stays within kGroupScratchBytes, and groups share one region.  An
+	// upscaled pass reads the TMEM snapshots its native pass (the round before)
+	// left in that round's scratch, so it never begins a group.
 	bool prep_ahead = false;
-	for (const auto &round : rounds) {
-		prep_ahead = prep_ahead || round.size() >= kOverlapMinPasses;
-		for (const PassRef &pr : round) prep_ahead = prep_ahead || pr.pass->scale_log2 != 0;
-	}
+	for (const auto &round : rounds) prep_ahead = prep_ahead || round.size() >= kOverlapMinPasses;
+	uint32_t num_passes = 0;
 	size_t off = 0, max_scratch = 0, scratch_base = 0;
 	for (size_t r = 0; r < rounds.size(); r++) {
 		// Work items carry the pass index above 17 bits of per-pass index.
 		if (rounds[r].size() > (1u << 15))
 			return set_error(RDP_MI_ERROR_UNSUPPORTED, "%zu passes in one round (at most 32768)", rounds[r].size());
 		RoundLayout &L = rl[r];
-		L.n_setup = L.n_span = L.n_tmem = L.n_tmem_gather = L.n_bin = L.n_raster = L.n_fill = L.n_quad = 0;
+		L.n_setup = L.n_span = L.n_scan = L.n_gather = L.n_bin = L.n_raster = L.n_fill = L.n_quad = 0;
+		L.first_pass = num_passes;
+		num_passes += (uint32_t)rounds[r].size();
 		L.n_dom_pre = L.n_dom_post = L.n_up = L.n_up_fill = L.n_resolve = 0;
 		for (uint32_t c = 0; c < kRasterClasses; c++) L.n_raster_class[c] = L.n_quad_class[c] = L.n_up_class[c] = 0;
-		size_t scr = scratch_base;
 		pl[r].resize(rounds[r].size());
+		size_t round_scratch = 0;
+		bool joins = false;  // an upscaled pass: in its native pass's group
+		for (size_t i = 0; i < rounds[r].size(); i++) {
+			pl[r][i].sl = scratch_layout(*rounds[r][i].pass);
+			round_scratch += pl[r][i].sl.total;
+			joins = joins || rounds[r][i].pass->scale_log2 != 0;
+		}
+		const bool fits = !groups.empty() && scratch_base + round_scratch <= kGroupScratchBytes &&
+		                  num_passes - rl[groups.back().first].first_pass <= kGroupMaxPasses;
+		if (prep_ahead || r == 0 || !(joins || fits)) {
+			groups.push_back({ r, 0, !prep_ahead });
+			if (!prep_ahead) scratch_base = 0;
+		}
+		Group &G = groups.back();
+		L.group = (uint32_t)groups.size() - 1;
+		// Shared TMEM replay: every upload of the group may run before every
+		// raster of it.
+		for (size_t q = G.first; q < r && G.tmem; q++) G.tmem = tmem_may_start_before(rounds, r, q);
+		G.rounds++;
+		size_t scr = scratch_base;
 		for (size_t i = 0; i < rounds[r].size(); i++) {
 			const HostPass &hp = *rounds[r][i].pass;
 			const uint32_t tx = (hp.fb_width + 7) / 8, ty = (hp.fb_height + 7) / 8;
@@ -755,9 +825,9 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 			L.n_span += (hp.num_tilerows + 7) / 8;
 			// An upscaled pass replays no uploads: it reads its native pass's
 			// TMEM snapshots.
-			if (!up) {
-				L.n_tmem += 8;
-				L.n_tmem_gather += 8 * tmem_blocks(hp.uploads.size());
+			if (!up && needs_tmem(rounds[r][i])) {
+				L.n_scan += 8;
+				L.n_gather += 8 * tmem_blocks(hp.uploads.size());
 			}
 			if (hp.domain_pre) L.n_dom_pre += domain_blocks(hp);
 			if (hp.domain_post) L.n_dom_post += domain_blocks(hp);
@@ -781,21 +851,11 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 					L.n_quad_class[std::min(hp.raster_class, kRasterClasses - 1)] += quads;
 				}
 			}
-			pi.sl = scratch_layout(hp);
 			pi.scratch_base = scr;
 			scr += pi.sl.total;
 		}
 		max_scratch = std::max(max_scratch, scr);
-		if (prep_ahead) scratch_base = align_up(scr, 256);
-		L.scratch = scr;
-		L.descs = off;
-		off = align_up(off + rounds[r].size() * sizeof(PassDesc), 256);
-		L.items_setup = off;
-		off = align_up(off + (L.n_setup + L.n_span) * 4ull, 256);
-		L.items_tmem = off;
-		off = align_up(off + (L.n_tmem + L.n_tmem_gather) * 4ull, 256);
-		L.items_bin = off;
-		off = align_up(off + L.n_bin * 4ull, 256);
+		scratch_base = align_up(scr, 256);
 		L.items_raster = off;
 		off = align_up(off + (L.n_raster + L.n_fill + L.n_quad) * 4ull, 256);
 		L.items_domain = off;
@@ -815,6 +875,20 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 			off = align_up(off + std::max<size_t>(hp.uploads.size(), 1) * sizeof(UploadInfo), 256);
 		}
 	}
+	// Descriptors and setup, span, bin and TMEM items of all rounds, each list
+	// in round order.
+	uint32_t n_setup = 0, n_span = 0, n_bin = 0, n_gather = 0, n_scan = 0;
+	for (const RoundLayout &L : rl) {
+		n_setup += L.n_setup;
+		n_span += L.n_span;
+		n_bin += L.n_bin;
+		n_gather += L.n_gather;
+		n_scan += L.n_scan;
+	}
+	const size_t off_descs = off;
+	off = align_up(off + num_passes * sizeof(PassDesc), 256);
+	const size_t off_prep = off;
+	off = align_up(off + ((size_t)n_setup + n_span + n_bin + n_gather + n_scan) * 4, 256);
 	const size_t total_input = off;
 	c.last_arena_bytes = total_input + max_scratch;
 
@@ -837,16 +911,25 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 	// Per processor: the TMEM snapshots of its pass in the round before, for
 	// an upscaled pass that follows it.
 	std::map<const Processor *, uint16_t *> native_tmem;
+	PassDesc *const all_descs = reinterpret_cast<PassDesc *>(h + off_descs);
+	uint32_t *const it_setup = reinterpret_cast<uint32_t *>(h + off_prep), *const it_span = it_setup + n_setup;
+	uint32_t *const it_bin = it_span + n_span, *const it_gather = it_bin + n_bin, *const it_scan = it_gather + n_gather;
+	auto on_device = [&](uint32_t *p) { return reinterpret_cast<const uint32_t *>(d + (reinterpret_cast<uint8_t *>(p) - h)); };
+	uint32_t ns = 0, nsp = 0, nb = 0, ntg = 0, nt = 0;  // items written so far
+	// Per processor: its last pass of the group with a TMEM scan.
+	std::map<const Processor *, uint32_t> tmem_last;
 	for (size_t r = 0; r < rounds.size(); r++) {
 		RoundLayout &L = rl[r];
-		PassDesc *descs = reinterpret_cast<PassDesc *>(h + L.descs);
-		uint32_t *it_setup = reinterpret_cast<uint32_t *>(h + L.items_setup);
-		uint32_t *it_tmem = reinterpret_cast<uint32_t *>(h + L.items_tmem);
-		uint32_t *it_bin = reinterpret_cast<uint32_t *>(h + L.items_bin);
+		PassDesc *descs = all_descs + L.first_pass;
+		const Group &G = groups[L.group];
+		const uint32_t group_pass = rl[G.first].first_pass;
+		if (r == G.first) tmem_last.clear();
 		uint32_t *it_raster = reinterpret_cast<uint32_t *>(h + L.items_raster);
 		uint32_t *it_domain = reinterpret_cast<uint32_t *>(h + L.items_domain);
 		uint32_t *it_up = reinterpret_cast<uint32_t *>(h + L.items_up);
-		uint32_t ns = 0, nsp = 0, nt = 0, ntg = 0, nb = 0, ndp = 0, ndq = 0, nrs = 0;
+		uint32_t ndp = 0, ndq = 0, nrs = 0;
+		uint32_t *const setup0 = it_setup + ns, *const span0 = it_span + nsp, *const bin0 = it_bin + nb;
+		uint32_t *const gather0 = it_gather + ntg, *const scan0 = it_scan + nt;
 		uint32_t upbase[kRasterClasses], nu[kRasterClasses];
 		for (uint32_t c = 0, acc = 0; c < kRasterClasses; c++) {
 			upbase[c] = acc;
@@ -865,27 +948,18 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 			qacc += L.n_quad_class[c];
 		}
 		Launch &LA = launches[r];
-		LA.descs = reinterpret_cast<const PassDesc *>(d + L.descs);
-		LA.items[0] = reinterpret_cast<const uint32_t *>(d + L.items_setup);
-		LA.items[1] = reinterpret_cast<const uint32_t *>(d + L.items_tmem);
-		LA.tmem_scan_items = LA.items[1] + L.n_tmem_gather;
-		LA.tmem_scan_n = L.n_tmem;
-		LA.span_items = LA.items[0] + L.n_setup;
-		LA.span_n = L.n_span;
-		LA.items[2] = reinterpret_cast<const uint32_t *>(d + L.items_bin);
-		LA.items[3] = reinterpret_cast<const uint32_t *>(d + L.items_raster);
-		LA.n[0] = L.n_setup;
-		LA.n[1] = L.n_tmem_gather;
-		LA.n[2] = L.n_bin;
-		LA.n[3] = L.n_raster;
-		LA.fill_items = LA.items[3] + L.n_raster;
+		memset(&LA, 0, sizeof(LA));
+		LA.descs = reinterpret_cast<const PassDesc *>(d + off_descs) + L.first_pass;
+		LA.prep_descs = reinterpret_cast<const PassDesc *>(d + off_descs) + group_pass;
+		const uint32_t *raster_items = reinterpret_cast<const uint32_t *>(d + L.items_raster);
+		LA.fill_items = raster_items + L.n_raster;
 		LA.fill_n = L.n_fill;
 		LA.prep_ahead = prep_ahead;
-		LA.tmem_early = tmem_may_start_early(rounds, r);
+		LA.tmem_early = prep_ahead && r > 0 && tmem_may_start_before(rounds, r, r - 1);
 		for (uint32_t c = 0; c < kRasterClasses; c++) {
-			LA.raster_items[c] = LA.items[3] + rbase[c];
+			LA.raster_items[c] = raster_items + rbase[c];
 			LA.raster_n[c] = L.n_raster_class[c];
-			LA.quad_items[c] = LA.items[3] + qbase[c];
+			LA.quad_items[c] = raster_items + qbase[c];
 			LA.quad_n[c] = L.n_quad_class[c];
 			LA.up_items[c] = reinterpret_cast<const uint32_t *>(d + L.items_up) + upbase[c];
 			LA.up_n[c] = L.n_up_class[c];
@@ -932,11 +1006,10 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 			D.spans = reinterpret_cast<SpanSetup *>(sb + pi.sl.setups);
 			D.tilerows = reinterpret_cast<uint32_t *>(sb + pi.sl.setups + pi.sl.spans);
 			D.bin_fine = reinterpret_cast<uint64_t *>(sb + pi.sl.setups + pi.sl.spans + pi.sl.tilerows);
-			D.tmem_blocks = reinterpret_cast<uint32_t *>(sb + pi.sl.setups + pi.sl.spans + pi.sl.tilerows + pi.sl.bins +
-			                                             pi.sl.tmem);
+			D.tmem_first = sb + pi.sl.setups + pi.sl.spans + pi.sl.tilerows + pi.sl.bins + pi.sl.tmem;
 			D.tmem_instances = reinterpret_cast<uint16_t *>(sb + pi.sl.setups + pi.sl.spans + pi.sl.tilerows + pi.sl.bins);
 			{
-				uint8_t *tail = sb + pi.sl.setups + pi.sl.spans + pi.sl.tilerows + pi.sl.bins + pi.sl.tmem + pi.sl.tmem_blocks;
+				uint8_t *tail = sb + pi.sl.setups + pi.sl.spans + pi.sl.tilerows + pi.sl.bins + pi.sl.tmem + pi.sl.tmem_first;
 				D.psetups = reinterpret_cast<PrimSetup *>(tail);
 				D.tilerow_prim = reinterpret_cast<uint16_t *>(tail + pi.sl.psetups);
 			}
@@ -981,16 +1054,23 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 				round_tmem[&pr] = D.tmem_instances;
 
 			const uint32_t pidx = (uint32_t)i;
-			for (uint32_t g = 0; g < (D.num_prims + 63) / 64; g++) it_setup[ns++] = (pidx << 7) | g;
-			for (uint32_t b = 0; b < (D.num_tilerows + 7) / 8; b++) it_setup[L.n_setup + nsp++] = (pidx << 17) | b;
-			if (!hp.scale_log2) {
-				for (uint32_t k = 0; k < 8; k++) it_tmem[L.n_tmem_gather + nt++] = (pidx << 12) | k;
+			const uint32_t gidx = L.first_pass - group_pass + pidx;  // in the group
+			for (uint32_t g = 0; g < (D.num_prims + 63) / 64; g++) it_setup[ns++] = (gidx << 7) | g;
+			for (uint32_t b = 0; b < (D.num_tilerows + 7) / 8; b++) it_span[nsp++] = (gidx << 17) | b;
+			if (!hp.scale_log2 && needs_tmem(rounds[r][i])) {
+				// A shared scan goes from a stream's pass to its next one.
+				auto last = G.tmem ? tmem_last.find(&pr) : tmem_last.end();
+				if (last != tmem_last.end())
+					all_descs[group_pass + last->second].tmem_next = gidx - last->second;
+				else
+					for (uint32_t k = 0; k < 8; k++) it_scan[nt++] = (gidx << 12) | k;
+				tmem_last[&pr] = gidx;
 				for (uint32_t b = 0; b < tmem_blocks(hp.uploads.size()); b++)
-					for (uint32_t k = 0; k < 8; k++) it_tmem[ntg++] = (pidx << 12) | (b << 3) | k;
+					for (uint32_t k = 0; k < 8; k++) it_gather[ntg++] = (gidx << 12) | (b << 3) | k;
 			}
 			if (D.num_prims) {
 				for (uint32_t y = 0; y < D.tiles_y; y++)
-					for (uint32_t g = 0; g < D.num_groups / 8; g++) it_bin[nb++] = (pidx << 17) | (y << 4) | g;
+					for (uint32_t g = 0; g < D.num_groups / 8; g++) it_bin[nb++] = (gidx << 17) | (y << 4) | g;
 			}
 			if (hp.domain_pre)
 				for (uint32_t b = 0; b < domain_blocks(hp); b++) it_domain[ndp++] = (pidx << 17) | b;
@@ -1000,14 +1080,37 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 				for (uint32_t b = 0; b < resolve_blocks(hp); b++)
 					it_domain[L.n_dom_pre + L.n_dom_post + nrs++] = (pidx << 17) | b;
 		}
-		// Setup, span and bin items: the passes above class 0 first.
+		LA.setup_items = on_device(setup0);
+		LA.span_items = on_device(span0);
+		LA.bin_items = on_device(bin0);
+		LA.gather_items = on_device(gather0);
+		LA.scan_items = on_device(scan0);
+		LA.setup_n = (uint32_t)(it_setup + ns - setup0);
+		LA.span_n = (uint32_t)(it_span + nsp - span0);
+		LA.bin_n = (uint32_t)(it_bin + nb - bin0);
+		LA.gather_n = (uint32_t)(it_gather + ntg - gather0);
+		LA.scan_n = (uint32_t)(it_scan + nt - scan0);
+		LA.group_tmem = G.tmem;
 		{
-			auto heavy = [&](uint32_t pidx) { return rounds[r][pidx].pass->raster_class > 0; };
-			LA.setup_hi = (uint32_t)(std::stable_partition(it_setup, it_setup + L.n_setup,
-			                                               [&](uint32_t it) { return heavy(it >> 7); }) - it_setup);
-			uint32_t *sp = it_setup + L.n_setup;
-			LA.span_hi = (uint32_t)(std::stable_partition(sp, sp + L.n_span, [&](uint32_t it) { return heavy(it >> 17); }) - sp);
-			LA.bin_hi = (uint32_t)(std::stable_partition(it_bin, it_bin + L.n_bin, [&](uint32_t it) { return heavy(it >> 17); }) - it_bin);
+			// The group's totals, at its first round.
+			Launch &F = launches[G.first];
+			F.group_rounds = (uint32_t)G.rounds;
+			F.group_setup += LA.setup_n;
+			F.group_span += LA.span_n;
+			F.group_bin += LA.bin_n;
+			F.group_gather += LA.gather_n;
+			F.group_scan += LA.scan_n;
+		}
+		// Setup, span and bin items that run ahead: the passes above class 0
+		// first.
+		if (prep_ahead) {
+			auto heavy = [&](uint32_t gidx) { return rounds[r][gidx].pass->raster_class > 0; };
+			LA.setup_hi = (uint32_t)(std::stable_partition(setup0, setup0 + LA.setup_n,
+			                                               [&](uint32_t it) { return heavy(it >> 7); }) - setup0);
+			LA.span_hi = (uint32_t)(std::stable_partition(span0, span0 + LA.span_n,
+			                                              [&](uint32_t it) { return heavy(it >> 17); }) - span0);
+			LA.bin_hi = (uint32_t)(std::stable_partition(bin0, bin0 + LA.bin_n,
+			                                             [&](uint32_t it) { return heavy(it >> 17); }) - bin0);
 		}
 		// Raster items, per class, passes with the most primitives per tile
 		// first: their tiles have the longest chains, so they start early
@@ -1057,7 +1160,10 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 		native_tmem = std::move(round_tmem);
 	}
 
-	HIP_CHECK(hipMemcpyAsync(d, h, total_input, hipMemcpyHostToDevice, c.stream));
+	if (staging.fixed)  // pageable
+		HIP_CHECK(hipMemcpyAsync(d, h, total_input, hipMemcpyHostToDevice, c.stream));
+	else
+		HIP_CHECK(launch_upload(h, d, total_input, c.stream));
 	HIP_CHECK(hipEventRecord(c.staging_done, c.stream));
 	c.staging_busy = true;
 	return 0;
@@ -1070,6 +1176,9 @@ struct Arenas {
 	DeviceBuffer *input, *scratch;
 	PinnedBuffer *staging;
 };
+
+// Passes of one processor in one plain submission.
+constexpr size_t kMaxPlainPasses = 64;
 
 static int submit_rounds(Lane &c, const std::vector<std::vector<PassRef>> &rounds, const Arenas *arenas = nullptr)
 {
@@ -1216,11 +1325,13 @@ static int submit_processors(Processor *const *procs, unsigned count, bool batch
 		// Keep each launch's pass count within the work-item encoding.
 		ret = submit_rounds(c, rounds, arenas);
 	} else {
-		// One pass per submission, except that an upscaled pass goes with its
-		// native pass: it reads the TMEM snapshots in that pass's scratch.
+		// One submission for a bounded number of passes, one pass per round: they
+		// share the copy of their inputs and their setup launches.  An upscaled
+		// pass goes with its native pass, whose TMEM snapshots it reads.
 		for (size_t k = 0; k < rounds.size() && !ret;) {
-			std::vector<std::vector<PassRef>> group{ rounds[k++] };
-			while (k < rounds.size() && rounds[k][0].pass->scale_log2) group.push_back(rounds[k++]);
+			std::vector<std::vector<PassRef>> group;
+			while (k < rounds.size() && (group.size() < kMaxPlainPasses || rounds[k][0].pass->scale_log2))
+				group.push_back(rounds[k++]);
 			ret = submit_rounds(c, group, arenas);
 		}
 	}

@@ -419,7 +419,7 @@ struct PassDesc {
 	SpanSetup *spans;
 	uint32_t *tilerows;        // per (prim, tile row): lo tile x | hi tile x << 16, 0xffff lo = empty
 	uint64_t *bin_fine;        // [tile][group] primitive masks
-	uint32_t *tmem_blocks;     // [block of kTmemBlock uploads][2048]: first write in block << 16 | value after it
+	uint8_t *tmem_first;       // [block of kTmemBlock uploads][2048]: the first upload of the block that writes the halfword
 	uint16_t *tmem_instances;  // (num_uploads + 1) x 2048 halfwords
 	PrimSetup *psetups;        // decoded edge and attribute setup per primitive
 	uint16_t *tilerow_prim;    // per tile-row entry: the primitive it belongs to
@@ -431,6 +431,7 @@ struct PassDesc {
 	uint32_t rdram_mask;       // rdram_size - 1
 	uint32_t num_prims;
 	uint32_t num_uploads;
+	uint32_t tmem_next;        // TMEM scan: passes from here to the same stream's next one in the launch (0: none)
 	uint32_t fb_addr, fb_width, fb_height, fb_fmt, depth_addr;
 	uint32_t tiles_x, tiles_y;
 	uint32_t num_spans;
