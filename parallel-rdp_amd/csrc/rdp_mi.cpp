@@ -41,6 +41,8 @@
 namespace rdp_mi {
 
 hipError_t launch_upload(const void *pinned, void *dst, size_t bytes, hipStream_t s);
+hipError_t launch_coherent_pull(const CopyRuns &, const void *staging, void *rdram, hipStream_t s);
+hipError_t launch_coherent_push(const CopyRuns &, const void *rdram, void *wmask, void *data, void *mask, hipStream_t s);
 hipError_t launch_prep(const PassDesc *, const uint32_t *setup, uint32_t, const uint32_t *span, uint32_t,
                        const uint32_t *gather, uint32_t, const uint32_t *scan, uint32_t, hipStream_t);
 hipError_t launch_bin(const PassDesc *, const uint32_t *, uint32_t, hipStream_t);
@@ -369,7 +371,10 @@ struct Processor {
 	// bytes the caller wrote meanwhile elsewhere in those pages survive.
 	bool coherent = false;
 	uint8_t *d_wmask = nullptr;
-	PinnedBuffer wb_data, wb_mask;
+	PinnedBuffer wb_data, wb_mask;   // RDRAM's layout, and a mask bit per byte of it
+	PinnedBuffer pull;               // pages on their way in, in RDRAM's layout
+	hipEvent_t pull_event = nullptr; // the device has read them
+	bool pull_pending = false;
 	std::vector<ByteRange> wb_runs;  // page runs of the write-back in flight
 	hipEvent_t wb_event = nullptr;
 	bool wb_pending = false;
@@ -1244,39 +1249,72 @@ static int coherent_complete(Processor &p)
 	std::lock_guard<std::mutex> g(p.wb_lock);
 	if (!p.wb_pending) return 0;
 	HIP_CHECK(hipEventSynchronize(p.wb_event));
-	uint8_t *host = p.user_rdram;
 	for (const ByteRange &r : p.wb_runs) {
-		const uint64_t *d = reinterpret_cast<const uint64_t *>(p.wb_data.ptr + r.lo);
-		const uint64_t *m = reinterpret_cast<const uint64_t *>(p.wb_mask.ptr + r.lo);
-		uint64_t *h = reinterpret_cast<uint64_t *>(host + r.lo);
-		for (uint64_t i = 0; i < (r.hi - r.lo) / 8; i++) {
-			uint64_t hv;
-			memcpy(&hv, h + i, 8);  // the caller's pointer may be unaligned
-			hv = (hv & ~m[i]) | (d[i] & m[i]);
-			memcpy(h + i, &hv, 8);
+		// 64 bytes per mask word: runs of all-ones words (most of a frame) in
+		// one copy each.
+		uint64_t whole = r.lo;  // everything from here to `at` is marked
+		for (uint64_t at = r.lo; at <= r.hi; at += 64) {
+			uint64_t m = 0;
+			if (at < r.hi) memcpy(&m, p.wb_mask.ptr + at / 8, 8);
+			if (m == ~0ull) continue;
+			if (at > whole) memcpy(p.user_rdram + whole, p.wb_data.ptr + whole, at - whole);
+			whole = at + 64;
+			for (; m; m &= m - 1) {
+				const int k = __builtin_ctzll(m);
+				p.user_rdram[at + k] = p.wb_data.ptr[at + k];
+			}
 		}
 	}
 	p.wb_pending = false;
 	return 0;
 }
 
-// Copy in the pages the passes read, before their launches.
+// Calls f(CopyRuns) for the runs, as many per call as a launch takes.
+template <typename F>
+static int for_copy_runs(const std::vector<ByteRange> &runs, F f)
+{
+	static_assert(kCoherentPage == 256 * 16, "a copy block is one page");
+	for (size_t i = 0; i < runs.size();) {
+		CopyRuns R;
+		memset(&R, 0, sizeof(R));
+		while (i < runs.size() && R.count < kCopyRuns) {
+			R.first[R.count] = (uint32_t)(runs[i].lo / 16);
+			R.units[R.count++] = (uint32_t)((runs[i].hi - runs[i].lo) / 16);
+			i++;
+		}
+		HIP_CHECK(f(R));
+	}
+	return 0;
+}
+
+// Copy the caller's pages to the device in stream order: into pinned staging
+// here, from there by a kernel (a copy from pageable memory pins its pages on
+// every call: 40-130 us for 300-600 KB, against 7 us for the copy and 15 for the
+// kernel).
+static int coherent_copy_in(Processor &p, const std::vector<ByteRange> &runs, hipStream_t st)
+{
+	if (runs.empty()) return 0;
+	if (p.pull_pending) {
+		HIP_CHECK(hipEventSynchronize(p.pull_event));
+		p.pull_pending = false;
+	}
+	for (const ByteRange &r : runs) memcpy(p.pull.ptr + r.lo, p.user_rdram + r.lo, r.hi - r.lo);
+	if (int err = for_copy_runs(runs, [&](const CopyRuns &R) { return launch_coherent_pull(R, p.pull.ptr, p.d_rdram, st); }))
+		return err;
+	HIP_CHECK(hipEventRecord(p.pull_event, st));
+	p.pull_pending = true;
+	return 0;
+}
+
+// Copy in the pages the passes read before they write them, before their
+// launches.
 static int coherent_pull(Processor &p, const std::vector<HostPass> &passes, hipStream_t st)
 {
 	if (int err = coherent_complete(p)) return err;
 	std::vector<ByteRange> ranges, runs;
-	for (const HostPass &hp : passes) {
-		pass_write_ranges(hp, ranges);
-		for (const UploadInfo &u : hp.uploads) {
-			ByteRange b;
-			if (!upload_read_range(u, b)) b = { 0, p.rdram_size };
-			ranges.push_back(b);
-		}
-	}
+	submission_read_ranges(passes, p.rdram_size, ranges);
 	page_runs(ranges, p.rdram_size, runs);
-	for (const ByteRange &r : runs)
-		HIP_CHECK(hipMemcpyAsync(p.d_rdram + r.lo, p.user_rdram + r.lo, r.hi - r.lo, hipMemcpyHostToDevice, st));
-	return 0;
+	return coherent_copy_in(p, runs, st);
 }
 
 // After the launches: copy out the written pages and their mask, clear the
@@ -1288,12 +1326,10 @@ static int coherent_push(Processor &p, const std::vector<HostPass> &passes, hipS
 	std::lock_guard<std::mutex> g(p.wb_lock);
 	page_runs(ranges, p.rdram_size, p.wb_runs);
 	if (p.wb_runs.empty()) return 0;
-	for (const ByteRange &r : p.wb_runs) {
-		const size_t n = r.hi - r.lo;
-		HIP_CHECK(hipMemcpyAsync(p.wb_data.ptr + r.lo, p.d_rdram + r.lo, n, hipMemcpyDeviceToHost, st));
-		HIP_CHECK(hipMemcpyAsync(p.wb_mask.ptr + r.lo, p.d_wmask + r.lo, n, hipMemcpyDeviceToHost, st));
-		HIP_CHECK(hipMemsetAsync(p.d_wmask + r.lo, 0, n, st));
-	}
+	if (int err = for_copy_runs(p.wb_runs, [&](const CopyRuns &R) {
+		    return launch_coherent_push(R, p.d_rdram, p.d_wmask, p.wb_data.ptr, p.wb_mask.ptr, st);
+	    }))
+		return err;
 	HIP_CHECK(hipEventRecord(p.wb_event, st));
 	p.wb_pending = true;
 	return 0;
@@ -2103,7 +2139,9 @@ int rdp_mi_create(rdp_mi_processor **out, void *rdram_ptr, size_t rdram_offset, 
 		if (p.d_wmask) (void)hipFree(p.d_wmask);
 		if (p.wb_data.ptr) (void)hipHostFree(p.wb_data.ptr);
 		if (p.wb_mask.ptr) (void)hipHostFree(p.wb_mask.ptr);
+		if (p.pull.ptr) (void)hipHostFree(p.pull.ptr);
 		if (p.wb_event) (void)hipEventDestroy(p.wb_event);
+		if (p.pull_event) (void)hipEventDestroy(p.pull_event);
 		delete h;
 		return set_error(code, "%s", msg);
 	};
@@ -2118,9 +2156,10 @@ int rdp_mi_create(rdp_mi_processor **out, void *rdram_ptr, size_t rdram_offset, 
 			return fail(RDP_MI_ERROR_OUT_OF_MEMORY, "RDRAM write mask allocation failed");
 		if (hipMemsetAsync(p.d_wmask, 0, rdram_size, c.stream) != hipSuccess)
 			return fail(RDP_MI_ERROR_DEVICE, "write mask clear failed");
-		if (p.wb_data.reserve(rdram_size) || p.wb_mask.reserve(rdram_size))
+		if (p.wb_data.reserve(rdram_size) || p.wb_mask.reserve(rdram_size / 8) || p.pull.reserve(rdram_size))
 			return fail(RDP_MI_ERROR_OUT_OF_MEMORY, "write-back buffers failed");
-		if (hipEventCreateWithFlags(&p.wb_event, hipEventDisableTiming) != hipSuccess)
+		if (hipEventCreateWithFlags(&p.wb_event, hipEventDisableTiming) != hipSuccess ||
+		    hipEventCreateWithFlags(&p.pull_event, hipEventDisableTiming) != hipSuccess)
 			return fail(RDP_MI_ERROR_DEVICE, "write-back event creation failed");
 		if (hipMemcpyAsync(p.d_rdram, p.user_rdram, rdram_size, hipMemcpyHostToDevice, c.stream) != hipSuccess)
 			return fail(RDP_MI_ERROR_DEVICE, "RDRAM upload failed");
@@ -2192,7 +2231,10 @@ void rdp_mi_destroy(rdp_mi_processor *h)
 		(void)hipFree(p.d_wmask);
 		(void)hipHostFree(p.wb_data.ptr);
 		(void)hipHostFree(p.wb_mask.ptr);
+		if (p.pull_pending) (void)hipEventSynchronize(p.pull_event);
+		(void)hipHostFree(p.pull.ptr);
 		(void)hipEventDestroy(p.wb_event);
+		(void)hipEventDestroy(p.pull_event);
 	}
 	delete h;
 }
@@ -2483,8 +2525,7 @@ static int scanout_queue(Processor &p, const rdp_mi_scanout_options &opts, uint3
 		vi_memory_range(p.vi, p.vi_regs, off, len);
 		std::vector<ByteRange> runs;
 		page_runs({ { off, (uint64_t)off + len } }, p.rdram_size, runs);
-		for (const ByteRange &r : runs)
-			HIP_CHECK(hipMemcpyAsync(p.d_rdram + r.lo, p.user_rdram + r.lo, r.hi - r.lo, hipMemcpyHostToDevice, c.stream));
+		if (int err = coherent_copy_in(p, runs, c.stream)) return err;
 	}
 	ViSource src;
 	src.rdram_size = p.rdram_size;

@@ -452,6 +452,14 @@ struct PassDesc {
 	uint8_t *resolve_rdram;  // an upscaled pass with DOMAIN_SSAA_RESOLVE: native RDRAM
 };
 
+// Runs of RDRAM a host-coherent copy covers, in units of 16 bytes (a kernel
+// argument).
+constexpr uint32_t kCopyRuns = 16;
+struct CopyRuns {
+	uint32_t count;
+	uint32_t first[kCopyRuns], units[kCopyRuns];
+};
+
 enum : uint32_t {
 	DOMAIN_SSAA_CLEAR = 1u << 0,    // the pre update also clears the write masks of the region
 	DOMAIN_SSAA_RESOLVE = 1u << 1,  // the upscaled raster records write masks; the pass is resolved
