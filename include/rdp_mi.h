@@ -115,7 +115,7 @@ void rdp_mi_enqueue_command_direct(rdp_mi_processor *p, unsigned num_words, cons
 
 /* Enqueue a packed run of complete commands through the command ring (no
  * reference counterpart: the reference's callers loop over enqueue_command,
- * which this performs with one ring hand-off per 64 Ki words).  Returns the
+ * which this performs with one ring hand-off per 4 Ki words).  Returns the
  * number of words consumed; a truncated trailing command is left unconsumed,
  * a word with an undefined or private opcode is skipped. */
 size_t rdp_mi_enqueue_command_list(rdp_mi_processor *p, size_t num_words, const uint32_t *words);

@@ -299,19 +299,54 @@ static Context &ctx()
 
 // Command ring of one processor (CommandRing, command_ring.cpp:31-134):
 // rdp_mi_enqueue_command copies complete commands in, and the processor's
-// ring thread takes everything available at once and decodes it.  Private
+// ring thread decodes them in place, a chunk at a time.  Long lists are handed
+// over in chunks, so decoding starts with the first and copying (block moves,
+// not word by word) never waits for the whole ring.  Private
 // meta commands ride in the same ring so they stay ordered with the RDP
 // commands (Op::MetaSignalTimeline and Op::MetaFlush, rdp_common.hpp:41-42).
 constexpr uint32_t kMetaSignal = 1, kMetaFlush = 2;
-constexpr size_t kRingWords = 1u << 16;
+// The ring holds a whole large frame (715 KB for 4096 textured triangles), so its
+// producer never sleeps in the middle of one; its pages are committed as used.
+constexpr size_t kRingWords = 1u << 18;
+constexpr size_t kRingChunk = 1u << 12;
+
+// Waits for something another thread or the GPU finishes within a frame poll
+// before they sleep: waking a thread whose core has gone idle took 50 us and more
+// here, two or three times a frame.  Callers poll for kWaitPollUs; a ring thread
+// without work for kRingPollUs, and only kRingPollers of them at a time, so that
+// many processors do not keep every core busy.
+constexpr int64_t kWaitPollUs = 1000, kRingPollUs = 400;
+constexpr int kRingPollers = 2;
+static std::atomic<int> g_ring_pollers{ 0 };
+template <typename Pred>
+static bool poll_for(int64_t us, Pred done)
+{
+	const auto t0 = std::chrono::steady_clock::now();
+	for (;;) {
+		for (int i = 0; i < 64; i++) {
+			if (done()) return true;
+			__builtin_ia32_pause();
+		}
+		if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(us)) return false;
+	}
+}
 
 struct CommandRing {
-	std::vector<uint32_t> words = std::vector<uint32_t>(kRingWords);
-	uint64_t write_count = 0, read_count = 0, completed_count = 0;
+	std::unique_ptr<uint32_t[]> words{ new uint32_t[kRingWords] };
+	// Words copied in, words decoded.  A chunk changes hands through these alone:
+	// under a common lock, the two threads put each other to sleep up to 18 times
+	// a frame.  `lock` is for sleeping and waking; a thread announces that it
+	// sleeps before it looks at the counts a last time, and the other one looks
+	// for that after it has changed them.
+	std::atomic<uint64_t> write_count{ 0 }, read_count{ 0 };
+	std::atomic<bool> sleeping{ false };  // the ring thread
+	std::atomic<int> waiters{ 0 };        // producers and drains
+	std::mutex push_lock;                 // one producer at a time
 	std::mutex lock;
-	std::condition_variable cv;  // data for the thread, space for producers, completion for drains
+	std::condition_variable cv;           // data for the ring thread
+	std::condition_variable progress;     // space for producers, completion for drains
 	std::thread thr;
-	bool stop = false;
+	std::atomic<bool> stop{ false };
 	bool pending = false;  // the processor held undelivered passes after the last batch
 };
 
@@ -345,7 +380,7 @@ struct Processor {
 	std::atomic<uint64_t> timeline{ 0 };
 	std::mutex tl_lock;
 	std::condition_variable tl_cv;
-	uint64_t timeline_done = 0;
+	std::atomic<uint64_t> timeline_done{ 0 };  // changed under tl_lock
 	int timeline_error = 0;
 	std::string timeline_error_msg;
 	// The first failed submission of the processor and its message.
@@ -1376,7 +1411,7 @@ static int submit_processors(Processor *const *procs, unsigned count, bool batch
 	if (ret == RDP_MI_ERROR_LIMIT && batched && arenas) return ret;
 	for (unsigned i = 0; i < count && !ret; i++)
 		if (procs[i]->coherent) ret = coherent_push(*procs[i], procs[i]->fe.completed(), c.stream);
-	for (unsigned i = 0; i < count; i++) procs[i]->fe.completed().clear();
+	for (unsigned i = 0; i < count; i++) procs[i]->fe.release_completed();
 	return ret;
 }
 
@@ -1544,9 +1579,10 @@ static unsigned ring_command_length(uint32_t w0)
 	return Frontend::command_length(w0);
 }
 
-// Decode complete commands in order (caller holds p.lock).  Completed passes
-// are handed to the device once enough queue up, bounding host memory.
-static void run_commands(Processor &p, const uint32_t *w, size_t n)
+// Decode complete commands in order (caller holds p.lock) and return the words
+// they take; an incomplete command at the end is left.  Completed passes are
+// handed to the device once enough queue up, bounding host memory.
+static size_t run_commands(Processor &p, const uint32_t *w, size_t n)
 {
 	size_t i = 0;
 	while (i < n) {
@@ -1567,6 +1603,21 @@ static void run_commands(Processor &p, const uint32_t *w, size_t n)
 		}
 		i += len;
 	}
+	return i;
+}
+
+// Decode the first commands of words [at, at + n) of the ring, which end with a
+// complete command: about kRingChunk words, so that producers get their space
+// back while decoding goes on (caller holds p.lock), from a flat copy in the
+// thread's own memory (14 us of 715 KB).  Returns the words taken.
+static size_t run_ring(Processor &p, const uint32_t *ring, uint64_t at, size_t n, uint32_t *local)
+{
+	const size_t pos = (size_t)(at & (kRingWords - 1));
+	n = std::min(n, kRingChunk);
+	const size_t flat = std::min(n, kRingWords - pos);
+	memcpy(local, ring + pos, flat * 4);
+	memcpy(local + flat, ring, (n - flat) * 4);
+	return run_commands(p, local, n);
 }
 
 // The ring thread (CommandRing::thread_loop, command_ring.cpp:86-134).  When
@@ -1575,41 +1626,52 @@ static void run_commands(Processor &p, const uint32_t *w, size_t n)
 static void ring_loop(Processor *p)
 {
 	CommandRing &r = *p->ring;
-	std::vector<uint32_t> batch;
+	std::vector<uint32_t> local(kRingChunk);
+	auto has_work = [&r] { return r.write_count != r.read_count || r.stop; };
 	for (;;) {
 		bool idle = false;
-		{
+		if (!has_work()) {
+			if (!r.pending) {
+				if (++g_ring_pollers <= kRingPollers) poll_for(kRingPollUs, has_work);
+				--g_ring_pollers;
+			}
 			std::unique_lock<std::mutex> g(r.lock);
-			auto has_work = [&r] { return r.write_count > r.read_count || r.stop; };
+			r.sleeping = true;
 			if (r.pending)
 				idle = !r.cv.wait_for(g, std::chrono::microseconds(500), has_work);
 			else
 				r.cv.wait(g, has_work);
-			if (!idle) {
-				if (r.write_count == r.read_count) break;  // stop requested, ring empty
-				const size_t n = (size_t)(r.write_count - r.read_count);
-				batch.resize(n);
-				for (size_t k = 0; k < n; k++) batch[k] = r.words[(r.read_count + k) & (kRingWords - 1)];
-				r.read_count += n;
-				r.cv.notify_all();  // space for producers
-			}
+			r.sleeping = false;
 		}
-		bool pending;
+		const uint64_t at = r.read_count;
+		size_t n = (size_t)(r.write_count - at);
+		if (!idle && n == 0) break;  // stop requested, ring empty
 		{
 			std::lock_guard<std::mutex> g(p->lock);
 			if (idle) {
 				if (!p->hold.load()) (void)submit_pending(*p);
 			} else
-				run_commands(*p, batch.data(), batch.size());
-			pending = !p->fe.completed().empty() && !p->hold.load();
+				n = run_ring(*p, r.words.get(), at, n, local.data());
+			r.pending = !p->fe.completed().empty() && !p->hold.load();
 		}
-		std::lock_guard<std::mutex> g(r.lock);
-		r.pending = pending;
-		if (!idle) {
-			r.completed_count = r.read_count;
-			r.cv.notify_all();  // drains
+		if (idle) continue;
+		r.read_count += n;
+		if (r.waiters) {
+			std::lock_guard<std::mutex> g(r.lock);
+			r.progress.notify_all();
 		}
 	}
+}
+
+// Waits until the ring thread has come as far as `reached` asks.
+template <typename Pred>
+static void ring_wait(CommandRing &r, Pred reached)
+{
+	if (poll_for(kWaitPollUs, reached)) return;
+	std::unique_lock<std::mutex> g(r.lock);
+	r.waiters++;
+	r.progress.wait(g, reached);
+	r.waiters--;
 }
 
 static CommandRing &ensure_ring(Processor &p)
@@ -1626,11 +1688,17 @@ static CommandRing &ensure_ring(Processor &p)
 static void ring_push(Processor &p, const uint32_t *w, size_t n)
 {
 	CommandRing &r = ensure_ring(p);
-	std::unique_lock<std::mutex> g(r.lock);
-	r.cv.wait(g, [&] { return r.write_count + n <= r.read_count + kRingWords; });
-	for (size_t k = 0; k < n; k++) r.words[(r.write_count + k) & (kRingWords - 1)] = w[k];
+	std::lock_guard<std::mutex> pg(r.push_lock);
+	if (r.write_count + n > r.read_count + kRingWords)
+		ring_wait(r, [&] { return r.write_count + n <= r.read_count + kRingWords; });
+	const size_t pos = (size_t)(r.write_count & (kRingWords - 1)), flat = std::min(n, kRingWords - pos);
+	memcpy(r.words.get() + pos, w, flat * 4);
+	memcpy(r.words.get(), w + flat, (n - flat) * 4);
 	r.write_count += n;
-	r.cv.notify_all();
+	if (r.sleeping) {
+		std::lock_guard<std::mutex> g(r.lock);
+		r.cv.notify_one();
+	}
 }
 
 // Wait until the ring thread has decoded everything enqueued so far
@@ -1643,8 +1711,20 @@ static void ring_drain(Processor &p)
 		r = p.ring.get();
 	}
 	if (!r) return;
-	std::unique_lock<std::mutex> g(r->lock);
-	r->cv.wait(g, [r] { return r->completed_count == r->write_count; });
+	const uint64_t end = r->write_count;
+	ring_wait(*r, [&] { return r->read_count >= end; });
+}
+
+// Whether the ring holds commands not decoded yet.
+static bool ring_busy(Processor &p)
+{
+	CommandRing *r;
+	{
+		std::lock_guard<std::mutex> g(p.ring_create);
+		r = p.ring.get();
+	}
+	if (!r) return false;
+	return r->read_count != r->write_count;
 }
 
 static bool has_ring(Processor &p)
@@ -2307,11 +2387,11 @@ size_t rdp_mi_enqueue_command_list(rdp_mi_processor *h, size_t num_words, const 
 		return i;
 	}
 	size_t i = 0, start = 0;
-	// Hand runs of complete commands to the ring, at most kRingWords at once;
+	// Hand runs of complete commands to the ring, at most kRingChunk words at once;
 	// words with an undefined or private opcode end a run and are skipped.
 	while (i < num_words) {
 		unsigned len = Frontend::command_length(words[i]);
-		if (len == 0 || i + len > num_words || i + len - start > kRingWords) {
+		if (len == 0 || i + len > num_words || i + len - start > kRingChunk) {
 			if (i > start) ring_push(h->p, words + start, i - start);
 			if (len != 0 && i + len > num_words) return i;
 			if (len == 0) i++;
@@ -2358,6 +2438,7 @@ int rdp_mi_wait_for_timeline_timeout(rdp_mi_processor *h, uint64_t value, uint64
 {
 	if (!h) return set_error(RDP_MI_ERROR_INVALID_ARGUMENT, "null processor");
 	Processor &p = h->p;
+	if (timeout_us >= (uint64_t)kWaitPollUs) poll_for(kWaitPollUs, [&] { return p.timeline_done >= value; });
 	std::unique_lock<std::mutex> g(p.tl_lock);
 	auto ready = [&] { return p.timeline_done >= value || p.timeline_error != 0; };
 	if (timeout_us == UINT64_MAX)
@@ -2512,9 +2593,21 @@ void rdp_mi_scanout_options_default(rdp_mi_scanout_options *o)
 static int scanout_queue(Processor &p, const rdp_mi_scanout_options &opts, uint32_t *out, unsigned *width,
                          unsigned *height, hipEvent_t done)
 {
-	ring_drain(p);
+	// A ring thread still decoding submits its own passes, with their words in
+	// its core's caches.
+	int failed_before;
+	{
+		std::lock_guard<std::mutex> g(p.lock);
+		failed_before = p.submit_error;
+	}
+	if (ring_busy(p)) {
+		const uint32_t w[1] = { kMetaFlush << 24 };
+		ring_push(p, w, 1);
+		ring_drain(p);
+	}
 	std::lock_guard<std::mutex> g(p.lock);
 	if (int err = flush_now(p)) return err;
+	if (p.submit_error && !failed_before) return set_error(p.submit_error, "%s", p.submit_error_msg.c_str());
 	Context &c = ctx();
 	std::lock_guard<std::mutex> lg(c.lock);
 	if (p.coherent) {
@@ -2741,7 +2834,7 @@ int rdp_mi_record(rdp_mi_processor *const *procs, unsigned count, int batched, r
 	std::vector<std::vector<PassRef>> rounds;
 	build_round_list(ps.data(), (unsigned)ps.size(), batched != 0, rounds);
 	int err = prepare_rounds(c, rounds, h->r.input, h->r.scratch, h->r.launches);
-	for (auto *p : ps) p->fe.completed().clear();
+	for (auto *p : ps) p->fe.release_completed();
 	if (!err && hipStreamSynchronize(c.stream) != hipSuccess) err = set_error(RDP_MI_ERROR_DEVICE, "upload failed");
 	if (err) {
 		delete h;
