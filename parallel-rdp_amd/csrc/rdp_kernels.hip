@@ -10,8 +10,9 @@
 //             reduces the per-8-line x extent into tile-row ranges; in blocks of
 //             their own, one lane per TMEM halfword carries values across the
 //             blocks of uploads, completing the TMEM snapshot after every upload.
-//   k_bin     one wave64 per (tile row, group of 64 primitives): a ballot per
-//             tile column produces the ordered 64-bit primitive masks.
+//   k_bin     one wave64 per (tile row, group of 64 primitives), eight per
+//             workgroup: an XOR prefix over the tile columns produces the ordered
+//             64-bit primitive masks.
 //   k_raster  one wave64 per 8x8 screen tile: colour/depth/coverage of the 64
 //             pixels live in registers while every binned primitive is shaded
 //             (coverage, interpolation, texturing, combiner) and merged (Z test,
@@ -610,86 +611,83 @@ void k_rows(const PassDesc *__restrict__ passes, const uint32_t *__restrict__ sc
 // ==========================================================================
 // Stage 3: binning.
 // ==========================================================================
-// One wave per (pass, tile row, block of 8 bin groups).  Primitive p of a
-// group covers the tile columns [lo_p, hi_p] of the row, so its bit is on in
-// the mask of column x iff lo_p <= x < hi_p + 1: XOR the bit into a
-// difference array at lo_p and hi_p + 1, and the inclusive XOR prefix over the
-// columns gives every column's mask.  Each lane then holds one column's masks
-// of the 8 groups and writes them as one 64-byte record (the group count is
-// padded to a multiple of 8, so the records are line aligned).
-DEV uint64_t xor_prefix64(uint64_t v, int lane)
+// One workgroup per (pass, tile row, block of 8 bin groups), a wave per group.
+// Primitive p of a group covers the tile columns [lo_p, hi_p] of the row, so its
+// bit is on in the mask of column x iff lo_p <= x < hi_p + 1: XOR the bit into a
+// difference array (in LDS) at lo_p and hi_p + 1, and the inclusive XOR prefix over
+// the columns gives every column's mask.  The 8 groups' masks of a column leave
+// as one 64-byte record (the group count is padded to a multiple of 8, so the
+// records are line aligned).
+//
+// A frame has a few hundred such blocks, so the launch is as long as one block's
+// chain: 64 groups by 60 rows took 13 us with one wave doing its 8 groups one after
+// another (three barriers and 12 LDS permutes each) and 5 us with a wave each
+// and the prefix in DPP moves.
+DEV uint32_t wave_xor_prefix(uint32_t v)
 {
-	uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
-#pragma unroll
-	for (int o = 1; o < 64; o <<= 1) {
-		const uint32_t tl = __shfl_up(lo, o, 64), th = __shfl_up(hi, o, 64);
-		if (lane >= o) {
-			lo ^= tl;
-			hi ^= th;
-		}
-	}
-	return ((uint64_t)hi << 32) | lo;
+	// Within rows of 16 lanes, then row 0 into 1 and 2 into 3, then both into 2, 3.
+	v ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);  // row_shr:1
+	v ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
+	v ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
+	v ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
+	v ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+	v ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+	return v;
 }
 
-__global__ __launch_bounds__(64) void k_bin(const PassDesc *__restrict__ passes, const uint32_t *__restrict__ items)
+DEV void wave_sync()
 {
-	__shared__ unsigned long long s_diff[65];
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__global__ __launch_bounds__(512) void k_bin(const PassDesc *__restrict__ passes, const uint32_t *__restrict__ items)
+{
+	__shared__ unsigned long long s_diff[8][65];
+	__shared__ uint64_t s_mask[64][9];  // [column][group], padded against bank conflicts
 	const uint32_t item = items[blockIdx.x];
 	const PassDesc &P = passes[item >> 17];
 	const uint32_t ty = (item >> 4) & 0x1fff, gb = (item & 0xf) * 8;
-	const int lane = threadIdx.x;
+	const uint32_t wave = uniform_u32(threadIdx.x >> 6), lane = threadIdx.x & 63;
 	const uint32_t tiles_x = P.tiles_x, G = P.num_groups;
-	const uint32_t real_groups = (P.num_prims + 63) / 64;
-	const uint32_t ng = real_groups > gb ? min(real_groups - gb, 8u) : 0u;
 
-	// Column range of each of the lane's 8 primitives in this tile row
-	// (lo > hi when the primitive misses the row).
-	uint32_t lo[8], hi[8];
-#pragma unroll
-	for (uint32_t k = 0; k < 8; k++) {
-		lo[k] = 0xffff;
-		hi[k] = 0;
-		const uint32_t prim = (gb + k) * 64 + (uint32_t)lane;
-		if (k < ng && prim < P.num_prims) {
-			const PrimRecord &r = P.prims[prim];
-			if (r.yhi >= r.ylo) {
-				const int row0 = r.ylo >> 3, row1 = r.yhi >> 3;
-				if ((int)ty >= row0 && (int)ty <= row1) {
-					const uint32_t v = P.tilerows[r.tilerow_offset + (ty - row0)];
-					lo[k] = v & 0xffff;
-					hi[k] = v >> 16;
-				}
+	// Column range of the lane's primitive in this tile row (lo > hi when the
+	// primitive misses the row).
+	uint32_t lo = 0xffff, hi = 0;
+	const uint32_t prim = (gb + wave) * 64 + lane;
+	if (prim < P.num_prims) {
+		const PrimRecord &r = P.prims[prim];
+		if (r.yhi >= r.ylo) {
+			const int row0 = r.ylo >> 3, row1 = r.yhi >> 3;
+			if ((int)ty >= row0 && (int)ty <= row1) {
+				const uint32_t v = P.tilerows[r.tilerow_offset + (ty - row0)];
+				lo = v & 0xffff;
+				hi = v >> 16;
 			}
 		}
 	}
 
 	uint64_t *out = P.bin_fine + (size_t)ty * tiles_x * G + gb;
 	for (uint32_t x0 = 0; x0 < tiles_x; x0 += 64) {
-		uint64_t m[8];
-#pragma unroll
-		for (uint32_t k = 0; k < 8; k++) {
-			m[k] = 0;
-			if (k >= ng) continue;
-			s_diff[lane] = 0;
-			if (lane == 0) s_diff[64] = 0;
-			__syncthreads();
-			// The part of [lo, hi] inside columns x0 .. x0 + 63.
-			const uint32_t a = max(lo[k], x0), b = min(hi[k], x0 + 63);
-			if (lo[k] <= hi[k] && a <= b) {
-				const unsigned long long bit = 1ull << lane;
-				atomicXor(&s_diff[a - x0], bit);
-				atomicXor(&s_diff[b + 1 - x0], bit);
-			}
-			__syncthreads();
-			m[k] = xor_prefix64(s_diff[lane], lane);
-			__syncthreads();
+		s_diff[wave][lane] = 0;
+		if (lane == 0) s_diff[wave][64] = 0;
+		wave_sync();
+		// The part of [lo, hi] inside columns x0 .. x0 + 63.
+		const uint32_t a = max(lo, x0), b = min(hi, x0 + 63);
+		if (lo <= hi && a <= b) {
+			const unsigned long long bit = 1ull << lane;
+			atomicXor(&s_diff[wave][a - x0], bit);
+			atomicXor(&s_diff[wave][b + 1 - x0], bit);
 		}
-		const uint32_t x = x0 + (uint32_t)lane;
-		if (x < tiles_x) {
-			uint64_t *o = out + (size_t)x * G;
-#pragma unroll
-			for (uint32_t k = 0; k < 8; k++) o[k] = m[k];
-		}
+		wave_sync();
+		const uint64_t d = s_diff[wave][lane];
+		const uint32_t m0 = wave_xor_prefix((uint32_t)d), m1 = wave_xor_prefix((uint32_t)(d >> 32));
+		s_mask[lane][wave] = ((uint64_t)m1 << 32) | m0;
+		__syncthreads();
+		const uint32_t x = threadIdx.x >> 3, g = threadIdx.x & 7;
+		if (x0 + x < tiles_x) out[(size_t)(x0 + x) * G + g] = s_mask[x][g];
+		__syncthreads();
 	}
 }
 
@@ -2690,7 +2688,7 @@ hipError_t launch_prep(const PassDesc *passes, const uint32_t *setup_items, uint
 hipError_t launch_bin(const PassDesc *passes, const uint32_t *items, uint32_t n, hipStream_t s)
 {
 	if (!n) return hipSuccess;
-	hipLaunchKernelGGL(k_bin, dim3(n), dim3(64), 0, s, passes, items);
+	hipLaunchKernelGGL(k_bin, dim3(n), dim3(512), 0, s, passes, items);
 	return hipGetLastError();
 }
 
