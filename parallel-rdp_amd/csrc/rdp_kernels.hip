@@ -2443,93 +2443,115 @@ void k_raster(const PassDesc *__restrict__ passes, const uint32_t *__restrict__ 
 // Passes whose every primitive is a FILL-mode primitive (variant 1, the
 // first row of the variant table).  A fill writes every channel of a pixel
 // it covers and reads neither colour nor depth, so the tile's framebuffer is
-// not loaded; a wave takes kFillTiles horizontally adjacent tiles, reads
-// their bin masks up front and runs them back to back.
+// not loaded; a wave takes kFillTiles horizontally adjacent tiles with the union
+// of their bin masks (coverage is the span's own test) and keeps the last covering
+// primitive's fill colour per sample.
+//
+// What bounds it is writing: the item's samples are dealt to the lanes along the
+// rows of one sample plane after another, so that a store covers runs of 32
+// pixels (natively), 16 (2x), 8 or 4.  Tile by tile, a store covered 8-pixel rows,
+// and in the sample planes runs of 4 pixels or fewer: the clears of 16 mixed
+// instances at 2x took 143 us that way and 48 us this way (22-36 VGPRs); natively
+// 32 instances take 26 us either way.
 constexpr uint32_t kFillTiles = kFillTilesPerItem;
-using FillVariant = RasterVariant<RAS_FILL | RAS_COPY, RAS_FILL, (int)COMB_ANY, TEXFMT_ANY, (int)DBP_ANY>;
+static_assert(kFillTiles == 4, "an item is 256 samples: four per lane");
 
 // UP: an upscaled pass's item (pass << 20 | tile group << 10 | tile row),
 // every lane a sample of its native pixel in the sample planes, as in
 // raster_tile.
 template <bool UP>
-DEV void fill_item(const PassDesc *__restrict__ passes, uint32_t item, uint16_t *s_unused)
+DEV void fill_item(const PassDesc *__restrict__ passes, uint32_t item)
 {
 	const PassDesc &P = passes[UP ? (item >> 20) : (item >> 14)];
 	const uint32_t tx0 = (UP ? (item >> 10) & 0x3ff : (item >> 7) & 0x7f) * kFillTiles, ty = UP ? item & 0x3ff : item & 0x7f;
-	const int lane = threadIdx.x & 63;
+	const uint32_t lane = threadIdx.x & 63;
 	const uint32_t fmt = P.fb_fmt;
-	const bool alias = P.fb_addr == P.depth_addr;
-	// Tiles start at multiples of 8, so a lane's sample slot (x mod S,
-	// y mod S) is the same in every tile of the item.
 	const int L = UP ? (int)uniform_u32(P.scale_log2) : 0;
-	const uint32_t smask = (1u << L) - 1;
-	const uint32_t slice = UP ? ((((uint32_t)lane >> 3) & smask) << L) + ((uint32_t)lane & smask) : 0;
-	const size_t plane8 = UP ? (size_t)slice * ((size_t)P.rdram_mask + 1) : 0;
-	const Mem m{ gptr(P.rdram) + plane8, gptr(P.hidden) + (plane8 >> 1), P.rdram_mask };
 	const AS_CONST RasterPrim *rprims = cptr(P.rprims);
-	const AS_CONST DrawState *states = cptr(P.states);
 	const AS_GLOBAL SpanSetup *spans = gptr(P.spans);
-	const AS_GLOBAL uint8_t *lut = (const AS_GLOBAL uint8_t *)g_blender_lut;
 	const AS_GLOBAL uint64_t *bins = gptr(P.bin_fine);
-	const Tex tex{ (const AS_LDS uint16_t *)(s_unused) };
 	const uint32_t G = P.num_groups, tiles_x = P.tiles_x;
-	const uint32_t y = ty * 8 + ((uint32_t)lane >> 3);
+	uint32_t addr_index;
+	switch (fmt) {
+	case FB_I4:
+	case FB_I8: addr_index = P.fb_addr; break;
+	case FB_RGBA5551:
+	case FB_IA88: addr_index = P.fb_addr >> 1; break;
+	default: addr_index = P.fb_addr >> 2; break;
+	}
 
-	uint64_t first[kFillTiles];
+	// The item's 32 x 8 samples are 32 / S x 8 / S native pixels in S^2 planes;
+	// sample number k * 64 + lane counts along the rows of plane 0, then plane 1.
+	// The native pixel of a lane is the same for every k of the upscaled factors.
+	const uint32_t wlog = 5 - L, plog = 8 - 2 * L;
+	uint32_t x[4], y[4], ci[4], color[4], covered = 0;
 #pragma unroll
-	for (uint32_t t = 0; t < kFillTiles; t++)
-		first[t] = tx0 + t < tiles_x && (uint32_t)lane < G ? bins[(size_t)(ty * tiles_x + tx0 + t) * G + lane] : 0;
-
+	for (uint32_t k = 0; k < 4; k++) {
+		const uint32_t n = k * 64 + lane, plane = n >> plog, r = n & ((1u << plog) - 1);
+		const uint32_t nx = ((tx0 * 8) >> L) + (r & ((1u << wlog) - 1)), ny = ((ty * 8) >> L) + (r >> wlog);
+		x[k] = (nx << L) + (plane & ((1u << L) - 1));
+		y[k] = (ny << L) + (plane >> L);
+		ci[k] = addr_index + (P.fb_width >> L) * ny + nx;
+		color[k] = 0;
+		// A sample outside the framebuffer is on no primitive's lines.
+		if (x[k] >= P.fb_width || y[k] >= P.fb_height) y[k] = 0x7fffffffu;
+	}
+	for (uint32_t gbase = 0; gbase < G; gbase += 64) {
+		uint64_t my_mask = 0;
 #pragma unroll
-	for (uint32_t t = 0; t < kFillTiles; t++) {
-		const uint32_t tx = tx0 + t;
-		if (tx >= tiles_x) break;
-		const uint32_t x = tx * 8 + ((uint32_t)lane & 7);
-		const bool in_fb = x < P.fb_width && y < P.fb_height;
-		uint32_t addr_index;
-		switch (fmt) {
-		case FB_I4:
-		case FB_I8: addr_index = P.fb_addr; break;
-		case FB_RGBA5551:
-		case FB_IA88: addr_index = P.fb_addr >> 1; break;
-		default: addr_index = P.fb_addr >> 2; break;
-		}
-		const uint32_t nx = x >> L, ny = y >> L;
-		const uint32_t ci = addr_index + (P.fb_width >> L) * ny + nx;
-		Pixel px;
-		px.c[0] = px.c[1] = px.c[2] = px.c[3] = 0;
-		px.depth = px.dz = 0;
-		px.dirty = 0;
-		for (uint32_t gbase = 0; gbase < G; gbase += 64) {
-			const uint64_t my_mask =
-			    gbase == 0 ? first[t] : (gbase + (uint32_t)lane < G ? bins[(size_t)(ty * tiles_x + tx) * G + gbase + lane] : 0);
-			uint64_t coarse = __ballot(my_mask != 0);
-			while (coarse) {
-				const int g = __ffsll((unsigned long long)coarse) - 1;
-				coarse &= coarse - 1;
-				const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)my_mask, g);
-				const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(my_mask >> 32), g);
-				uint64_t mask = ((uint64_t)hi << 32) | lo;
-				while (mask) {
-					const int bit = __ffsll((unsigned long long)mask) - 1;
-					mask &= mask - 1;
-					const AS_CONST RasterPrim *ps = rprims + ((gbase + (uint32_t)g) * 64 + (uint32_t)bit);
-					const RasterPrimHead h = ldc(reinterpret_cast<const AS_CONST RasterPrimHead *>(&ps->ylo));
-					if (!in_fb || (int)y < h.ylo || (int)y > h.yhi) continue;
-					raster_prim<FillVariant>(ps, h, states, spans, tex, lut, fmt, alias, ci, (int)x, (int)y, px, L);
-				}
+		for (uint32_t t = 0; t < kFillTiles; t++)
+			if (tx0 + t < tiles_x && gbase + lane < G) my_mask |= bins[(size_t)(ty * tiles_x + tx0 + t) * G + gbase + lane];
+		uint64_t coarse = __ballot(my_mask != 0);
+		while (coarse) {
+			const int g = __ffsll((unsigned long long)coarse) - 1;
+			coarse &= coarse - 1;
+			const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)my_mask, g);
+			const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(my_mask >> 32), g);
+			uint64_t mask = ((uint64_t)hi << 32) | lo;
+			while (mask) {
+				const int bit = __ffsll((unsigned long long)mask) - 1;
+				mask &= mask - 1;
+				const AS_CONST RasterPrim *ps = rprims + ((gbase + (uint32_t)g) * 64 + (uint32_t)bit);
+				const RasterPrimHead h = ldc(reinterpret_cast<const AS_CONST RasterPrimHead *>(&ps->ylo));
+				// shading.h:45-52: a native-resolution primitive shades every
+				// sample as its pixel's first one.
+				const uint32_t snap = L && (ps->flags & TRI_DISABLE_UPSCALING) ? ~((1u << L) - 1) : ~0u;
+#pragma unroll
+				for (uint32_t k = 0; k < 4; k++)
+					if ((int)y[k] >= h.ylo && (int)y[k] <= h.yhi) {
+						// The row's last 16 bytes: base_x, start_x, end_x, lodlength | valid.
+						const AS_GLOBAL uint32_t *row =
+						    (const AS_GLOBAL uint32_t *)(spans + (h.span_offset + ((y[k] & snap) - (uint32_t)h.ylo))) + 12;
+						const int start_x = (int)row[1], end_x = (int)row[2], xs = (int)(x[k] & snap);
+						if ((row[3] >> 16) && xs >= start_x && xs <= end_x) {
+							color[k] = h.fill_color;
+							covered |= 1u << k;
+						}
+					}
 			}
 		}
-		if (in_fb && (px.dirty & PIXEL_COLOR_DIRTY)) {
-			store_color(m, fmt, ci, px);
-			if (P.wmask) mark_color(gptr(P.wmask), P.rdram_mask, fmt, ci);
+	}
+	// A fill writes no depth field (with colour and depth aliased the colour store
+	// is the depth store).
+	if (fmt == FB_I4) covered = 0;  // fills do not write 4-bit images
+	uint32_t written = covered ? 1u : 0u;
+#pragma unroll
+	for (uint32_t k = 0; k < 4; k++)
+		if (covered & (1u << k)) {
+			const size_t plane8 = UP ? (size_t)((k * 64 + lane) >> plog) * ((size_t)P.rdram_mask + 1) : 0;
+			const Mem m{ gptr(P.rdram) + plane8, gptr(P.hidden) + (plane8 >> 1), P.rdram_mask };
+			Pixel px;
+			px.dirty = 0;
+			fill_pixel(px, fmt, false, ci[k], color[k]);
+			store_color(m, fmt, ci[k], px);
+			if (P.wmask) mark_color(gptr(P.wmask), P.rdram_mask, fmt, ci[k]);
 		}
-		// A fill writes no depth field (with colour and depth aliased the
-		// colour store is the depth store).
-		if constexpr (UP) {
-			if (P.domain_flags & DOMAIN_SSAA_RESOLVE)
-				emit_scaled_write_masks(P.up_wmask, ny * (P.fb_width >> L) + nx, in_fb ? px.dirty & PIXEL_COLOR_DIRTY : 0u, L,
-				                        lane);
+	if constexpr (UP) {
+		// One write-mask bit per native pixel: lanes that are 1 << plog apart hold
+		// its other samples.
+		if (P.domain_flags & DOMAIN_SSAA_RESOLVE) {
+			for (uint32_t d = 1u << plog; d < 64; d <<= 1) written |= (uint32_t)__shfl_xor((int)written, (int)d, 64);
+			if (written && lane < (1u << plog)) atomicOr(P.up_wmask + (ci[0] - addr_index), 1u);
 		}
 	}
 }
@@ -2537,20 +2559,14 @@ DEV void fill_item(const PassDesc *__restrict__ passes, uint32_t item, uint16_t 
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8)))
 void k_raster_fill(const PassDesc *__restrict__ passes, const uint32_t *__restrict__ items, int32_t xcd_chunk)
 {
-	__shared__ uint16_t s_unused[2];
-	// Fill-mode primitives never divide; the table is filled all the same so
-	// every kernel that can reach perspective_divide has it.
-	persp_table_init();
-	fill_item<false>(passes, items[xcd_local_item(blockIdx.x, gridDim.x, xcd_chunk)], s_unused);
+	fill_item<false>(passes, items[xcd_local_item(blockIdx.x, gridDim.x, xcd_chunk)]);
 }
 
 // The FILL-only passes of an upscaled round: k_raster_fill in the sample planes.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8)))
 void k_raster_fill_up(const PassDesc *__restrict__ passes, const uint32_t *__restrict__ items, int32_t xcd_chunk)
 {
-	__shared__ uint16_t s_unused[2];
-	persp_table_init();
-	fill_item<true>(passes, items[xcd_local_item(blockIdx.x, gridDim.x, xcd_chunk)], s_unused);
+	fill_item<true>(passes, items[xcd_local_item(blockIdx.x, gridDim.x, xcd_chunk)]);
 }
 
 // One launch for every raster work item of a round (persistent): the grid
@@ -2575,7 +2591,7 @@ void k_raster_round(const PassDesc *__restrict__ passes, const uint32_t *__restr
 		else if (k < n_hi + n_lo)
 			raster_tile<CLS, false>(passes, items_lo[k - n_hi], s_tmem);
 		else
-			fill_item<false>(passes, fill_items[k - n_hi - n_lo], s_tmem);
+			fill_item<false>(passes, fill_items[k - n_hi - n_lo]);
 		// The next item's staging must not overwrite texels this item's
 		// lanes still read.
 		__syncthreads();
