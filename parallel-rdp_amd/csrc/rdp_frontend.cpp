@@ -84,43 +84,12 @@ void Frontend::complete_pass(HostPass &&p, uint32_t domain_height)
 		done.push_back(std::move(p));
 }
 
-// At most this many emptied passes are kept, and none whose words alone hold
-// more than kSpareWords (passes end at 8192 primitives of at most 44 words).
-constexpr size_t kSparePasses = 4, kSpareWords = 1u << 19;
-
-void Frontend::release_completed()
-{
-	for (HostPass &p : done) {
-		if (spare.size() == kSparePasses) break;
-		if (p.words.capacity() > kSpareWords) continue;
-		HostPass e;
-		e.words.swap(p.words);
-		e.states.swap(p.states);
-		e.prims.swap(p.prims);
-		e.uploads.swap(p.uploads);
-		e.words.clear();
-		e.states.clear();
-		e.prims.clear();
-		e.uploads.clear();
-		spare.push_back(std::move(e));
-	}
-	done.clear();
-}
-
-HostPass Frontend::fresh_pass()
-{
-	if (spare.empty()) return HostPass();
-	HostPass p = std::move(spare.back());
-	spare.pop_back();
-	return p;
-}
-
 void Frontend::flush()
 {
 	const uint32_t dh = std::max(domain_height, ref_domain_height());
 	if (!cur.empty()) complete_pass(std::move(cur), dh);
 	domain_height = 0;
-	cur = fresh_pass();
+	cur = HostPass();
 	state_dirty = true;
 	color_write_pending = false;
 	depth_write_pending = false;
@@ -133,10 +102,10 @@ void Frontend::flush()
 // S * ylo .. S * yhi + S - 1 per primitive (span_setup.comp:89-95), an
 // S-times framebuffer, no TMEM uploads of its own (it reads the native
 // pass's TMEM snapshots).
-HostPass Frontend::upscaled_copy(const HostPass &n)
+HostPass Frontend::upscaled_copy(const HostPass &n) const
 {
 	const int32_t S = 1 << scale_log2;
-	HostPass u = fresh_pass();
+	HostPass u;
 	u.words = n.words;
 	u.states = n.states;
 	u.prims = n.prims;

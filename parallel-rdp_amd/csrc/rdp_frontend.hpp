@@ -102,12 +102,8 @@ public:
 	// Close the open pass (if it holds any work).
 	void flush();
 
-	// Completed passes, in order.
+	// Completed passes, in order; the caller takes ownership.
 	std::vector<HostPass> &completed() { return done; }
-	// Drops the completed passes and keeps the storage of a few for the next
-	// ones: a frame's command words grow to hundreds of KB, and growing and
-	// faulting that memory in again took as long as decoding into it.
-	void release_completed();
 
 	bool has_pending_work() const { return !done.empty() || !cur.empty(); }
 
@@ -162,8 +158,6 @@ private:
 	// Upscaled domain rows of the reference passes that ended inside cur.
 	uint32_t domain_height = 0;
 	std::vector<HostPass> done;
-	std::vector<HostPass> spare;  // emptied, kSparePasses at most
-	HostPass fresh_pass();
 	RefPassState ref;
 	std::function<void(uint32_t, const char *)> validation;
 
@@ -179,7 +173,7 @@ private:
 	void ref_pass_end();
 	void split_at_last_mark();
 	void split_or_flush();
-	HostPass upscaled_copy(const HostPass &native);
+	HostPass upscaled_copy(const HostPass &native) const;
 	uint32_t ref_domain_height() const;
 	void complete_pass(HostPass &&p, uint32_t domain_height);
 	void validate_draw() const;

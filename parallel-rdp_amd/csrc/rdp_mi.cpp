@@ -305,9 +305,11 @@ static Context &ctx()
 // meta commands ride in the same ring so they stay ordered with the RDP
 // commands (Op::MetaSignalTimeline and Op::MetaFlush, rdp_common.hpp:41-42).
 constexpr uint32_t kMetaSignal = 1, kMetaFlush = 2;
-// The ring holds a whole large frame (715 KB for 4096 textured triangles), so its
-// producer never sleeps in the middle of one; its pages are committed as used.
-constexpr size_t kRingWords = 1u << 18;
+// 256 KB stay in the two cores' caches.  (A ring that holds a whole frame, 1 MB,
+// and word vectors kept from frame to frame cost 130 us of a 640x480 two-cycle
+// frame, 515 against 385 us, on a busy host: each frame then walks memory that
+// has left the caches, where the allocator hands out what was just freed.)
+constexpr size_t kRingWords = 1u << 16;
 constexpr size_t kRingChunk = 1u << 12;
 
 // Waits for something another thread or the GPU finishes within a frame poll
@@ -1411,7 +1413,7 @@ static int submit_processors(Processor *const *procs, unsigned count, bool batch
 	if (ret == RDP_MI_ERROR_LIMIT && batched && arenas) return ret;
 	for (unsigned i = 0; i < count && !ret; i++)
 		if (procs[i]->coherent) ret = coherent_push(*procs[i], procs[i]->fe.completed(), c.stream);
-	for (unsigned i = 0; i < count; i++) procs[i]->fe.release_completed();
+	for (unsigned i = 0; i < count; i++) procs[i]->fe.completed().clear();
 	return ret;
 }
 
@@ -2834,7 +2836,7 @@ int rdp_mi_record(rdp_mi_processor *const *procs, unsigned count, int batched, r
 	std::vector<std::vector<PassRef>> rounds;
 	build_round_list(ps.data(), (unsigned)ps.size(), batched != 0, rounds);
 	int err = prepare_rounds(c, rounds, h->r.input, h->r.scratch, h->r.launches);
-	for (auto *p : ps) p->fe.release_completed();
+	for (auto *p : ps) p->fe.completed().clear();
 	if (!err && hipStreamSynchronize(c.stream) != hipSuccess) err = set_error(RDP_MI_ERROR_DEVICE, "upload failed");
 	if (err) {
 		delete h;
