@@ -299,7 +299,7 @@ static Context &ctx()
 
 // Command ring of one processor (CommandRing, command_ring.cpp:31-134):
 // rdp_mi_enqueue_command copies complete commands in, and the processor's
-// ring thread decodes them in place, a chunk at a time.  Long lists are handed
+// ring thread decodes them, a chunk at a time.  Long lists are handed
 // over in chunks, so decoding starts with the first and copying (block moves,
 // not word by word) never waits for the whole ring.  Private
 // meta commands ride in the same ring so they stay ordered with the RDP

@@ -82,7 +82,7 @@ constexpr int kTileSize = 8;                 // 8x8 pixel screen tile = one wave
 constexpr int kMaxPrimsPerPass = 8192;       // 128 bin groups x 64 primitives
 constexpr int kBinGroups = kMaxPrimsPerPass / 64;
 constexpr int kMaxUploadsPerPass = 1023;     // TMEM snapshots per pass (4 KiB each)
-// Uploads one lane of the TMEM gather applies in a row (k_tmem_gather).  The lane
+// Uploads one lane of the TMEM gather applies in a row (k_prep).  The lane
 // is a serial chain of divisions and RDRAM reads, 0.9 us per upload, and a frame
 // has few blocks; the scan walks the blocks.  64 uploads of one frame: gather 28 us
 // with blocks of 32, 16 of 16, 9 of 8, 6 of 4; the scan 4.6 us up to 8 and 7 of 4.
