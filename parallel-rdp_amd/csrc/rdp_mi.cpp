@@ -44,8 +44,8 @@ hipError_t launch_upload(const void *pinned, void *dst, size_t bytes, hipStream_
 hipError_t launch_coherent_pull(const CopyRuns &, const void *staging, void *rdram, hipStream_t s);
 hipError_t launch_coherent_push(const CopyRuns &, const void *rdram, void *wmask, void *data, void *mask, hipStream_t s);
 hipError_t launch_prep(const PassDesc *, const uint32_t *setup, uint32_t, const uint32_t *span, uint32_t,
-                       const uint32_t *gather, uint32_t, const uint32_t *scan, uint32_t, hipStream_t);
-hipError_t launch_bin(const PassDesc *, const uint32_t *, uint32_t, hipStream_t);
+                       const uint32_t *gather, uint32_t, const uint32_t *scan, uint32_t, bool beside, hipStream_t);
+hipError_t launch_bin(const PassDesc *, const uint32_t *, uint32_t, bool beside, hipStream_t);
 hipError_t launch_raster(uint32_t cls, const PassDesc *, const uint32_t *, uint32_t, int32_t, bool, hipStream_t);
 hipError_t launch_raster_fill(const PassDesc *, const uint32_t *, uint32_t, int32_t, hipStream_t);
 hipError_t launch_raster_round(uint32_t cls, const PassDesc *, const uint32_t *, uint32_t, const uint32_t *, uint32_t,
@@ -621,6 +621,18 @@ static uint64_t framebuffer_bytes(const HostPass &hp)
 // series too.
 constexpr uint32_t kOverlapMinPasses = 8;
 
+static hipError_t launch_setup(const Launch &L, const uint32_t *setup, uint32_t n_setup, const uint32_t *span,
+                               uint32_t n_span, hipStream_t st)
+{
+	return launch_prep(L.prep_descs, setup, n_setup, span, n_span, nullptr, 0, nullptr, 0, L.prep_ahead, st);
+}
+
+static hipError_t launch_tmem(const Launch &L, uint32_t n_gather, uint32_t n_scan, hipStream_t st)
+{
+	return launch_prep(L.prep_descs, nullptr, 0, nullptr, 0, L.gather_items, n_gather, L.scan_items, n_scan, L.prep_ahead,
+	                   st);
+}
+
 static int execute_launches(const std::vector<Launch> &launches, Lane &lane, const LaunchConfig &cfg,
                             hipEvent_t *stage_events = nullptr, hipEvent_t *raster_events = nullptr)
 {
@@ -634,12 +646,12 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 		for (size_t r = 0; r < launches.size(); r++) {
 			const Launch &L = launches[r];
 			// The heavier classes' passes first (prep_heavy), then the rest.
-			HIP_CHECK(launch_prep(L.prep_descs, L.setup_items, L.setup_hi, L.span_items, L.span_hi, nullptr, 0, nullptr, 0, prep));
-			HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.bin_hi, prep));
+			HIP_CHECK(launch_setup(L, L.setup_items, L.setup_hi, L.span_items, L.span_hi, prep));
+			HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.bin_hi, L.prep_ahead, prep));
 			HIP_CHECK(hipEventRecord(lane.events[r].prep_heavy, prep));
-			HIP_CHECK(launch_prep(L.prep_descs, L.setup_items + L.setup_hi, L.setup_n - L.setup_hi, L.span_items + L.span_hi,
-			                      L.span_n - L.span_hi, nullptr, 0, nullptr, 0, prep));
-			HIP_CHECK(launch_bin(L.prep_descs, L.bin_items + L.bin_hi, L.bin_n - L.bin_hi, prep));
+			HIP_CHECK(launch_setup(L, L.setup_items + L.setup_hi, L.setup_n - L.setup_hi, L.span_items + L.span_hi,
+			                       L.span_n - L.span_hi, prep));
+			HIP_CHECK(launch_bin(L.prep_descs, L.bin_items + L.bin_hi, L.bin_n - L.bin_hi, L.prep_ahead, prep));
 			HIP_CHECK(hipEventRecord(lane.events[r].prep_done, prep));
 		}
 	}
@@ -648,9 +660,6 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 		const Launch &L = launches[r];
 		const bool big = ahead && L.passes >= kOverlapMinPasses;
 		const bool fork_tmem = big && L.scan_n;
-		auto launch_tmem = [&](hipStream_t st) {
-			return launch_prep(L.prep_descs, nullptr, 0, nullptr, 0, L.gather_items, L.gather_n, L.scan_items, L.scan_n, st);
-		};
 		// Raster launches after the class floor: the merged light launch and
 		// the heavier classes.
 		const uint32_t lo = std::min(cfg.min_class, kRasterClasses - 1);
@@ -679,33 +688,33 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 			hipEvent_t after = E.fork;
 			if (early) after = (r == 1 && ahead && prev_tmem_forked) ? lane.start : lane.events[r - 1].pre_raster;
 			HIP_CHECK(hipStreamWaitEvent(side, after, 0));
-			HIP_CHECK(launch_tmem(side));
+			HIP_CHECK(launch_tmem(L, L.gather_n, L.scan_n, side));
 			HIP_CHECK(hipEventRecord(E.tmem_done, side));
 		}
 		prev_tmem_forked = fork_tmem || !L.scan_n;
 		if (ahead) {
-			if (!fork_tmem) HIP_CHECK(launch_tmem(s));
+			if (!fork_tmem) HIP_CHECK(launch_tmem(L, L.gather_n, L.scan_n, s));
 			HIP_CHECK(hipStreamWaitEvent(s, E.prep_done, 0));
 			HIP_CHECK(hipEventRecord(E.pre_raster, s));
 		} else if (stage_events) {
 			if (L.group_rounds)
-				HIP_CHECK(launch_prep(L.prep_descs, L.setup_items, L.group_setup, L.span_items, L.group_span, nullptr, 0, nullptr, 0, s));
+				HIP_CHECK(launch_setup(L, L.setup_items, L.group_setup, L.span_items, L.group_span, s));
 			HIP_CHECK(hipEventRecord(stage_events[r * 4 + 0], s));
 			if (!L.group_tmem)
-				HIP_CHECK(launch_tmem(s));
+				HIP_CHECK(launch_tmem(L, L.gather_n, L.scan_n, s));
 			else if (L.group_rounds)
-				HIP_CHECK(launch_prep(L.prep_descs, nullptr, 0, nullptr, 0, L.gather_items, L.group_gather, L.scan_items, L.group_scan, s));
+				HIP_CHECK(launch_tmem(L, L.group_gather, L.group_scan, s));
 			HIP_CHECK(hipEventRecord(stage_events[r * 4 + 1], s));
-			if (L.group_rounds) HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.group_bin, s));
+			if (L.group_rounds) HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.group_bin, L.prep_ahead, s));
 			HIP_CHECK(hipEventRecord(stage_events[r * 4 + 2], s));
 		} else {
 			if (L.group_rounds) {
 				const uint32_t gather = L.group_tmem ? L.group_gather : 0, scan = L.group_tmem ? L.group_scan : 0;
-				HIP_CHECK(launch_prep(L.prep_descs, L.setup_items, L.group_setup, L.span_items, L.group_span, L.gather_items, gather,
-				                      L.scan_items, scan, s));
-				HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.group_bin, s));
+				HIP_CHECK(launch_prep(L.prep_descs, L.setup_items, L.group_setup, L.span_items, L.group_span, L.gather_items,
+				                      gather, L.scan_items, scan, L.prep_ahead, s));
+				HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.group_bin, L.prep_ahead, s));
 			}
-			if (!L.group_tmem) HIP_CHECK(launch_tmem(s));
+			if (!L.group_tmem) HIP_CHECK(launch_tmem(L, L.gather_n, L.scan_n, s));
 		}
 		// The domain's pre update reads native RDRAM before this round's
 		// raster writes it (submit_render_pass, rdp_renderer.cpp:2240-2246).
