@@ -107,3 +107,29 @@ def test_tmem_replay_order_through_server():
     for out, s in zip(outs, streams):
         total, lines = harness.compare(out, harness.run_oracle(s))
         assert total == 0, f"{s.name}: " + "; ".join(lines)
+
+
+@pytest.mark.parametrize("sources", ["pass_a", "other"])
+def test_replays_of_one_recording(sources):
+    """The replay of round 1's TMEM, first in the graph or behind round 0's raster:
+    graph replays and direct launches in turn, each from fresh contents."""
+    import rdp_mi
+    streams = [texture_stream(300 + i, sources == "pass_a") for i in range(9)]
+    print(f"[case] four replays of 9 render-to-texture streams, sources={sources}", flush=True)
+    refs = [harness.run_oracle(s) for s in streams]
+    procs = [rdp_mi.CommandProcessor(rs.RDRAM_SIZE) for _ in streams]
+    for p, s in zip(procs, streams):
+        p.hold_submissions()
+        p.enqueue_commands(s.frames[0].words)
+    rec = rdp_mi.Recording(procs, batched=True)
+    for graph in (True, False, True, True):
+        for p, s in zip(procs, streams):
+            p.write_rdram(s.rdram_init)
+            p.write_hidden_rdram(np.full(rs.RDRAM_SIZE // 2, s.hidden_init, np.uint8))
+        rec.replay(1, use_graph=graph)
+        for p, s, ref in zip(procs, streams, refs):
+            total, lines = harness.compare((p.read_rdram(), p.read_hidden_rdram(), p.read_tmem()), ref)
+            assert total == 0, f"{s.name}: " + "; ".join(lines)
+    rec.close()
+    for p in procs:
+        p.close()
