@@ -805,6 +805,14 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 constexpr size_t kGroupScratchBytes = 64u << 20;
 constexpr uint32_t kGroupMaxPasses = 1u << 12;
 
+// From this size on a serving lane's packed inputs go through the copy engine: the
+// upload kernel's waves would take slots on the GPU from the other lanes' rasters
+// for as long as PCIe takes (3 lanes at 40000 frames/s, batches of 5 to 9 frames
+// with 0.3 MB each: p50 latency 1.17 ms with the kernel, 0.80 from 1 MB on, 0.73 from
+// 512 KB on; GPU time 0.49, 0.29 and 0.28).  Smaller ones, and submissions that have
+// the GPU to themselves, gain from the kernel (launch_upload).
+constexpr size_t kLaneCopyBytes = 1u << 19;
+
 // Pack the inputs of all rounds into `input` (one async copy on the context
 // stream) and describe the launches.  Caller holds the context lock.
 static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &rounds, DeviceBuffer &input,
@@ -1231,7 +1239,8 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 		native_tmem = std::move(round_tmem);
 	}
 
-	if (staging.fixed)  // pageable
+	// A fixed staging array is pageable.
+	if (staging.fixed || (&c != &ctx() && total_input >= kLaneCopyBytes))
 		HIP_CHECK(hipMemcpyAsync(d, h, total_input, hipMemcpyHostToDevice, c.stream));
 	else
 		HIP_CHECK(launch_upload(h, d, total_input, c.stream));
