@@ -2754,12 +2754,12 @@ hipError_t launch_coherent_push(const CopyRuns &R, const void *rdram, void *wmas
 
 // Setup (n_setup items of 64 primitives, then n_span of 8 tile-row entries)
 // and TMEM replay (n_gather and n_scan items of 256 halfwords); either may be
-// absent.  beside: rasters run at the same time.
+// absent.  wave_blocks: see Launch.
 hipError_t launch_prep(const PassDesc *passes, const uint32_t *setup_items, uint32_t n_setup, const uint32_t *span_items,
                        uint32_t n_span, const uint32_t *gather_items, uint32_t n_gather, const uint32_t *scan_items,
-                       uint32_t n_scan, bool beside, hipStream_t s)
+                       uint32_t n_scan, bool wave_blocks, hipStream_t s)
 {
-	if (beside) {
+	if (wave_blocks) {
 		if (n_gather) hipLaunchKernelGGL(k_tmem_gather, dim3(n_gather), dim3(256), 0, s, passes, gather_items);
 		if (n_setup) hipLaunchKernelGGL(k_setup, dim3(n_setup), dim3(64), 0, s, passes, setup_items);
 		if (n_scan) hipLaunchKernelGGL(k_tmem_scan, dim3(n_scan), dim3(256), 0, s, passes, scan_items);
@@ -2775,10 +2775,10 @@ hipError_t launch_prep(const PassDesc *passes, const uint32_t *setup_items, uint
 	return hipGetLastError();
 }
 
-hipError_t launch_bin(const PassDesc *passes, const uint32_t *items, uint32_t n, bool beside, hipStream_t s)
+hipError_t launch_bin(const PassDesc *passes, const uint32_t *items, uint32_t n, bool wave_blocks, hipStream_t s)
 {
 	if (!n) return hipSuccess;
-	if (beside)
+	if (wave_blocks)
 		hipLaunchKernelGGL(k_bin_wave, dim3(n), dim3(64), 0, s, passes, items);
 	else
 		hipLaunchKernelGGL(k_bin, dim3(n), dim3(512), 0, s, passes, items);

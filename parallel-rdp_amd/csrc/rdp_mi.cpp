@@ -44,8 +44,8 @@ hipError_t launch_upload(const void *pinned, void *dst, size_t bytes, hipStream_
 hipError_t launch_coherent_pull(const CopyRuns &, const void *staging, void *rdram, hipStream_t s);
 hipError_t launch_coherent_push(const CopyRuns &, const void *rdram, void *wmask, void *data, void *mask, hipStream_t s);
 hipError_t launch_prep(const PassDesc *, const uint32_t *setup, uint32_t, const uint32_t *span, uint32_t,
-                       const uint32_t *gather, uint32_t, const uint32_t *scan, uint32_t, bool beside, hipStream_t);
-hipError_t launch_bin(const PassDesc *, const uint32_t *, uint32_t, bool beside, hipStream_t);
+                       const uint32_t *gather, uint32_t, const uint32_t *scan, uint32_t, bool wave_blocks, hipStream_t);
+hipError_t launch_bin(const PassDesc *, const uint32_t *, uint32_t, bool wave_blocks, hipStream_t);
 hipError_t launch_raster(uint32_t cls, const PassDesc *, const uint32_t *, uint32_t, int32_t, bool, hipStream_t);
 hipError_t launch_raster_fill(const PassDesc *, const uint32_t *, uint32_t, int32_t, hipStream_t);
 hipError_t launch_raster_round(uint32_t cls, const PassDesc *, const uint32_t *, uint32_t, const uint32_t *, uint32_t,
@@ -507,6 +507,10 @@ struct Launch {
 	const uint32_t *resolve_items;  // the round's upscaled passes with a resolve, after their raster
 	uint32_t resolve_n;
 	bool prep_ahead;  // a round of many passes is present: every round has its own scratch, setup/binning run ahead
+	// How a submission with prep_ahead is laid out (launch_plan): setup, span and
+	// bin launches in blocks of one wave; setup one round ahead of the rasters
+	// instead of all of it first; round 1's early TMEM replay before everything.
+	bool wave_blocks, staggered, tmem1_first;
 	bool tmem_early;  // no upload reads what the previous round's raster writes
 	uint64_t raster_bytes;  // algorithmic framebuffer bytes read + written by k_raster
 	uint64_t class_bytes[kRasterClasses], fill_bytes;  // the same per raster launch
@@ -602,10 +606,10 @@ static uint64_t framebuffer_bytes(const HostPass &hp)
 
 // Launches every round on the lane's stream.  In submissions with a round of
 // many passes, three streams share the work:
-//   - `prep` runs the setup and binning of every round ahead, starting with
-//     the submission (they read only the packed inputs, and each round has
-//     its own scratch region), so round r+1's setup overlaps round r's
-//     raster;
+//   - `prep` runs the setup and binning of every round ahead (they read only
+//     the packed inputs, and each round has its own scratch region), all of it
+//     from the submission's start or one round ahead (launch_plan), so round
+//     r+1's setup overlaps round r's raster;
 //   - `side` runs a round's TMEM replay, which depends on RDRAM as the
 //     previous round left it and writes only its own snapshots, beside the
 //     rest of the round, and then the raster launches of the heavier
@@ -621,15 +625,43 @@ static uint64_t framebuffer_bytes(const HostPass &hp)
 // series too.
 constexpr uint32_t kOverlapMinPasses = 8;
 
+// The layout of a submission with a round of at least kOverlapMinPasses passes.
+// A captured graph puts its branches on a few queues by the order in which they
+// were launched, and two branches on one queue wait for each other; direct
+// launches gain or lose little by any of this.  Graph replays of mixed streams, ms
+// without / with (instances x frames, two rounds a frame):
+//   - Blocks of one wave: 24x1 0.275 / 0.268, 64x1 0.571 / 0.534, 64x4 2.53 /
+//     2.48, but 12x1 0.207 / 0.218: small launches need no room beside a raster.
+//   - Round 1's TMEM replay first: of more than two rounds, together with the next
+//     item; of two 64x1 the same, 96x1 0.874 / 0.858, 64 streams of 1250
+//     triangles 0.867 / 0.839, but 32x1 0.318 / 0.335.
+//   - Setup one round ahead: 32x8 2.88 / 2.84, 64x4 2.53 / 2.48, 10x6 0.754 /
+//     0.730, 8x8 0.883 / 0.806, but 8x2 0.318 / 0.340.
+//   - With upscaled passes the rasters are milliseconds long and all three cost
+//     (64 streams at 4x 10.66 / 10.73, 2x with readback 3.16 / 3.22; 12x2 at 2x
+//     1.25 / 1.45 with the setup one round ahead).
+struct LaunchPlan {
+	bool wave_blocks, staggered, tmem1_first;
+};
+static LaunchPlan launch_plan(size_t rounds, size_t widest, bool upscaled)
+{
+	LaunchPlan p = {};
+	if (upscaled || widest < kOverlapMinPasses) return p;
+	p.wave_blocks = widest >= 24;
+	p.staggered = rounds > 4 || (rounds > 2 && widest >= 24);
+	p.tmem1_first = p.staggered || (rounds == 2 && widest >= 64);
+	return p;
+}
+
 static hipError_t launch_setup(const Launch &L, const uint32_t *setup, uint32_t n_setup, const uint32_t *span,
                                uint32_t n_span, hipStream_t st)
 {
-	return launch_prep(L.prep_descs, setup, n_setup, span, n_span, nullptr, 0, nullptr, 0, L.prep_ahead, st);
+	return launch_prep(L.prep_descs, setup, n_setup, span, n_span, nullptr, 0, nullptr, 0, L.wave_blocks, st);
 }
 
 static hipError_t launch_tmem(const Launch &L, uint32_t n_gather, uint32_t n_scan, hipStream_t st)
 {
-	return launch_prep(L.prep_descs, nullptr, 0, nullptr, 0, L.gather_items, n_gather, L.scan_items, n_scan, L.prep_ahead,
+	return launch_prep(L.prep_descs, nullptr, 0, nullptr, 0, L.gather_items, n_gather, L.scan_items, n_scan, L.wave_blocks,
 	                   st);
 }
 
@@ -648,37 +680,40 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 		for (uint32_t c = lo + 1; c < kRasterClasses; c++) n += L.rn(c, cfg.quad);
 		return n;
 	};
-	// Round 1's early TMEM replay needs nothing of the submission, and where round
-	// 0 (clears) leaves the side stream empty it is the first thing launched: in a
-	// captured graph a branch further back in the order shares a queue with round
-	// 0's raster and waits for it.  64 streams: the replay began 73 us into the step
-	// and the heavy raster 188, instead of 0 and 80; 0.867 against 0.841 ms.
+	// Round 1's early TMEM replay needs nothing of the submission; it may come
+	// first where round 0 (clears) leaves the side stream empty.
 	bool tmem1_first = false;
 	if (ahead) {
 		HIP_CHECK(hipEventRecord(lane.start, s));
-		tmem1_first = launches.size() > 1 && launches[1].passes >= kOverlapMinPasses && launches[1].scan_n &&
-		              launches[1].tmem_early && !launches[0].scan_n && !heavy_tiles(launches[0]);
+		tmem1_first = launches[0].tmem1_first && launches.size() > 1 && launches[1].passes >= kOverlapMinPasses &&
+		              launches[1].scan_n && launches[1].tmem_early && !launches[0].scan_n && !heavy_tiles(launches[0]);
 		if (tmem1_first) {
 			HIP_CHECK(hipStreamWaitEvent(side, lane.start, 0));
 			HIP_CHECK(launch_tmem(launches[1], launches[1].gather_n, launches[1].scan_n, side));
 			HIP_CHECK(hipEventRecord(lane.events[1].tmem_done, side));
 		}
 		HIP_CHECK(hipStreamWaitEvent(prep, lane.start, 0));
-		for (size_t r = 0; r < launches.size(); r++) {
-			const Launch &L = launches[r];
-			// The heavier classes' passes first (prep_heavy), then the rest.
-			HIP_CHECK(launch_setup(L, L.setup_items, L.setup_hi, L.span_items, L.span_hi, prep));
-			HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.bin_hi, L.prep_ahead, prep));
-			HIP_CHECK(hipEventRecord(lane.events[r].prep_heavy, prep));
-			HIP_CHECK(launch_setup(L, L.setup_items + L.setup_hi, L.setup_n - L.setup_hi, L.span_items + L.span_hi,
-			                       L.span_n - L.span_hi, prep));
-			HIP_CHECK(launch_bin(L.prep_descs, L.bin_items + L.bin_hi, L.bin_n - L.bin_hi, L.prep_ahead, prep));
-			HIP_CHECK(hipEventRecord(lane.events[r].prep_done, prep));
-		}
 	}
+	// Setup and binning of round r on the prep stream: the heavier classes' passes
+	// first (prep_heavy), then the rest.
+	auto prep_round = [&](size_t r) -> int {
+		const Launch &L = launches[r];
+		HIP_CHECK(launch_setup(L, L.setup_items, L.setup_hi, L.span_items, L.span_hi, prep));
+		HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.bin_hi, L.wave_blocks, prep));
+		HIP_CHECK(hipEventRecord(lane.events[r].prep_heavy, prep));
+		HIP_CHECK(launch_setup(L, L.setup_items + L.setup_hi, L.setup_n - L.setup_hi, L.span_items + L.span_hi,
+		                       L.span_n - L.span_hi, prep));
+		HIP_CHECK(launch_bin(L.prep_descs, L.bin_items + L.bin_hi, L.bin_n - L.bin_hi, L.wave_blocks, prep));
+		HIP_CHECK(hipEventRecord(lane.events[r].prep_done, prep));
+		return 0;
+	};
+	size_t prepped = 0;
 	bool prev_tmem_forked = false;
 	for (size_t r = 0; r < launches.size(); r++) {
 		const Launch &L = launches[r];
+		if (ahead)
+			while (prepped < launches.size() && (!L.staggered || prepped <= r + (r > 0)))
+				if (int err = prep_round(prepped++)) return err;
 		const bool big = ahead && L.passes >= kOverlapMinPasses;
 		const bool fork_tmem = big && L.scan_n;
 		uint32_t merged = 0;
@@ -725,14 +760,14 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 			else if (L.group_rounds)
 				HIP_CHECK(launch_tmem(L, L.group_gather, L.group_scan, s));
 			HIP_CHECK(hipEventRecord(stage_events[r * 4 + 1], s));
-			if (L.group_rounds) HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.group_bin, L.prep_ahead, s));
+			if (L.group_rounds) HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.group_bin, L.wave_blocks, s));
 			HIP_CHECK(hipEventRecord(stage_events[r * 4 + 2], s));
 		} else {
 			if (L.group_rounds) {
 				const uint32_t gather = L.group_tmem ? L.group_gather : 0, scan = L.group_tmem ? L.group_scan : 0;
 				HIP_CHECK(launch_prep(L.prep_descs, L.setup_items, L.group_setup, L.span_items, L.group_span, L.gather_items,
-				                      gather, L.scan_items, scan, L.prep_ahead, s));
-				HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.group_bin, L.prep_ahead, s));
+				                      gather, L.scan_items, scan, L.wave_blocks, s));
+				HIP_CHECK(launch_bin(L.prep_descs, L.bin_items, L.group_bin, L.wave_blocks, s));
 			}
 			if (!L.group_tmem) HIP_CHECK(launch_tmem(L, L.gather_n, L.scan_n, s));
 		}
@@ -857,8 +892,14 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 	// stays within kGroupScratchBytes, and groups share one region.  An
 	// upscaled pass reads the TMEM snapshots its native pass (the round before)
 	// left in that round's scratch, so it never begins a group.
-	bool prep_ahead = false;
-	for (const auto &round : rounds) prep_ahead = prep_ahead || round.size() >= kOverlapMinPasses;
+	bool upscaled = false;
+	size_t widest = 0;
+	for (const auto &round : rounds) {
+		widest = std::max(widest, round.size());
+		for (const PassRef &pr : round) upscaled = upscaled || pr.pass->scale_log2 != 0;
+	}
+	const bool prep_ahead = widest >= kOverlapMinPasses;
+	const LaunchPlan plan = launch_plan(rounds.size(), widest, upscaled);
 	uint32_t num_passes = 0;
 	size_t off = 0, max_scratch = 0, scratch_base = 0;
 	for (size_t r = 0; r < rounds.size(); r++) {
@@ -1034,6 +1075,9 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 		LA.fill_items = raster_items + L.n_raster;
 		LA.fill_n = L.n_fill;
 		LA.prep_ahead = prep_ahead;
+		LA.wave_blocks = plan.wave_blocks;
+		LA.staggered = plan.staggered;
+		LA.tmem1_first = plan.tmem1_first;
 		LA.tmem_early = prep_ahead && r > 0 && tmem_may_start_before(rounds, r, r - 1);
 		for (uint32_t c = 0; c < kRasterClasses; c++) {
 			LA.raster_items[c] = raster_items + rbase[c];

@@ -24,11 +24,11 @@ def test_bins_match_oracle(width, height, prims):
 
 
 def test_bins_of_a_wide_batch_match_oracle():
-    """Eight processors and more in a round: setup, spans and bins in blocks of
-    one wave, beside the raster."""
+    """24 processors and more in a round: setup, spans and bins in blocks of one
+    wave, beside the raster."""
     import rdp_mi
-    streams = [rs.config0_stream(seed=width * 1000 + prims + 1, num_triangles=prims, width=width, height=height)
-               for width, height, prims in SIZES + [(64, 64, 1), (320, 240, 4160)]]
+    streams = [rs.config0_stream(seed=width * 1000 + prims + 1 + 7 * k, num_triangles=prims, width=width, height=height)
+               for k, (width, height, prims) in enumerate(2 * SIZES + [(64, 64, 1), (320, 240, 4160)] + 6 * [(40, 40, 70)])]
     print(f"[case] {len(streams)} processors in one batch", flush=True)
     procs = [rdp_mi.CommandProcessor(rs.RDRAM_SIZE) for _ in streams]
     for p, s in zip(procs, streams):

@@ -109,27 +109,35 @@ def test_tmem_replay_order_through_server():
         assert total == 0, f"{s.name}: " + "; ".join(lines)
 
 
+# Two rounds a frame: where a submission's layout changes with its passes a round
+# and its rounds (blocks of one wave from 24 passes on, setup one round ahead from 3
+# or 5 rounds on, the replay of round 1's TMEM first from 64 passes or 3 rounds on).
+@pytest.mark.parametrize("procs,frames", [(9, 1), (8, 2), (23, 1), (24, 1), (8, 3), (24, 2), (64, 1)])
 @pytest.mark.parametrize("sources", ["pass_a", "other"])
-def test_replays_of_one_recording(sources):
-    """The replay of round 1's TMEM, first in the graph or behind round 0's raster:
-    graph replays and direct launches in turn, each from fresh contents."""
+def test_replays_of_one_recording(sources, procs, frames):
+    """Graph replays and direct launches in turn, each from fresh contents."""
     import rdp_mi
-    streams = [texture_stream(300 + i, sources == "pass_a") for i in range(9)]
-    print(f"[case] four replays of 9 render-to-texture streams, sources={sources}", flush=True)
+    streams = []
+    for i in range(procs):
+        parts = [texture_stream(300 + i + 1000 * f, sources == "pass_a") for f in range(frames)]
+        streams.append(rs.Stream(name=f"rtt{i}", seed=i, frames=[p.frames[0] for p in parts], rdram_init=parts[0].rdram_init,
+                                 hidden_init=3))
+    print(f"[case] {procs} processors, {2 * frames} rounds, sources={sources}", flush=True)
     refs = [harness.run_oracle(s) for s in streams]
-    procs = [rdp_mi.CommandProcessor(rs.RDRAM_SIZE) for _ in streams]
-    for p, s in zip(procs, streams):
+    ps = [rdp_mi.CommandProcessor(rs.RDRAM_SIZE) for _ in streams]
+    for p, s in zip(ps, streams):
         p.hold_submissions()
-        p.enqueue_commands(s.frames[0].words)
-    rec = rdp_mi.Recording(procs, batched=True)
+        p.enqueue_commands(s.all_words())
+    rec = rdp_mi.Recording(ps, batched=True)
+    assert rec.rounds == 2 * frames
     for graph in (True, False, True, True):
-        for p, s in zip(procs, streams):
+        for p, s in zip(ps, streams):
             p.write_rdram(s.rdram_init)
             p.write_hidden_rdram(np.full(rs.RDRAM_SIZE // 2, s.hidden_init, np.uint8))
         rec.replay(1, use_graph=graph)
-        for p, s, ref in zip(procs, streams, refs):
+        for p, s, ref in zip(ps, streams, refs):
             total, lines = harness.compare((p.read_rdram(), p.read_hidden_rdram(), p.read_tmem()), ref)
-            assert total == 0, f"{s.name}: " + "; ".join(lines)
+            assert total == 0, f"{s.name}, graph {graph}: " + "; ".join(lines)
     rec.close()
-    for p in procs:
+    for p in ps:
         p.close()
