@@ -34,6 +34,7 @@
 #include "rdp_dump.hpp"
 #include "rdp_frontend.hpp"
 #include "rdp_hazard.hpp"
+#include "rdp_ring.hpp"
 #include "rdp_types.hpp"
 #include "rdp_vi.hpp"
 #include "rdp_view.hpp"
@@ -296,61 +297,6 @@ static Context &ctx()
 	static Context c;
 	return c;
 }
-
-// Command ring of one processor (CommandRing, command_ring.cpp:31-134):
-// rdp_mi_enqueue_command copies complete commands in, and the processor's
-// ring thread decodes them, a chunk at a time.  Long lists are handed
-// over in chunks, so decoding starts with the first and copying (block moves,
-// not word by word) never waits for the whole ring.  Private
-// meta commands ride in the same ring so they stay ordered with the RDP
-// commands (Op::MetaSignalTimeline and Op::MetaFlush, rdp_common.hpp:41-42).
-constexpr uint32_t kMetaSignal = 1, kMetaFlush = 2;
-// 256 KB stay in the two cores' caches.  (A ring that holds a whole frame, 1 MB,
-// and word vectors kept from frame to frame cost 130 us of a 640x480 two-cycle
-// frame, 515 against 385 us, on a busy host: each frame then walks memory that
-// has left the caches, where the allocator hands out what was just freed.)
-constexpr size_t kRingWords = 1u << 16;
-constexpr size_t kRingChunk = 1u << 12;
-
-// Waits for something another thread or the GPU finishes within a frame poll
-// before they sleep: waking a thread whose core has gone idle took 50 us and more
-// here, two or three times a frame.  Callers poll for kWaitPollUs; a ring thread
-// without work for kRingPollUs, and only kRingPollers of them at a time, so that
-// many processors do not keep every core busy.
-constexpr int64_t kWaitPollUs = 1000, kRingPollUs = 400;
-constexpr int kRingPollers = 2;
-static std::atomic<int> g_ring_pollers{ 0 };
-template <typename Pred>
-static bool poll_for(int64_t us, Pred done)
-{
-	const auto t0 = std::chrono::steady_clock::now();
-	for (;;) {
-		for (int i = 0; i < 64; i++) {
-			if (done()) return true;
-			__builtin_ia32_pause();
-		}
-		if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(us)) return false;
-	}
-}
-
-struct CommandRing {
-	std::unique_ptr<uint32_t[]> words{ new uint32_t[kRingWords] };
-	// Words copied in, words decoded.  A chunk changes hands through these alone:
-	// under a common lock, the two threads put each other to sleep up to 18 times
-	// a frame.  `lock` is for sleeping and waking; a thread announces that it
-	// sleeps before it looks at the counts a last time, and the other one looks
-	// for that after it has changed them.
-	std::atomic<uint64_t> write_count{ 0 }, read_count{ 0 };
-	std::atomic<bool> sleeping{ false };  // the ring thread
-	std::atomic<int> waiters{ 0 };        // producers and drains
-	std::mutex push_lock;                 // one producer at a time
-	std::mutex lock;
-	std::condition_variable cv;           // data for the ring thread
-	std::condition_variable progress;     // space for producers, completion for drains
-	std::thread thr;
-	std::atomic<bool> stop{ false };
-	bool pending = false;  // the processor held undelivered passes after the last batch
-};
 
 struct Processor {
 	Frontend fe;
@@ -1690,159 +1636,58 @@ static size_t run_commands(Processor &p, const uint32_t *w, size_t n)
 	return i;
 }
 
-// Decode the first commands of words [at, at + n) of the ring, which end with a
-// complete command: about kRingChunk words, so that producers get their space
-// back while decoding goes on (caller holds p.lock), from a flat copy in the
-// thread's own memory (14 us of 715 KB).  Returns the words taken.
-static size_t run_ring(Processor &p, const uint32_t *ring, uint64_t at, size_t n, uint32_t *local)
-{
-	const size_t pos = (size_t)(at & (kRingWords - 1));
-	n = std::min(n, kRingChunk);
-	const size_t flat = std::min(n, kRingWords - pos);
-	memcpy(local, ring + pos, flat * 4);
-	memcpy(local + flat, ring, (n - flat) * 4);
-	return run_commands(p, local, n);
-}
+// What the processor's ring thread does with commands.
+struct RingSink {
+	Processor &p;
 
-// The ring thread (CommandRing::thread_loop, command_ring.cpp:86-134).  When
-// no command arrives for 500 us while passes are waiting, it hands them to
-// the device (the reference's MetaIdle).
-static void ring_loop(Processor *p)
-{
-	CommandRing &r = *p->ring;
-	std::vector<uint32_t> local(kRingChunk);
-	auto has_work = [&r] { return r.write_count != r.read_count || r.stop; };
-	for (;;) {
-		bool idle = false;
-		if (!has_work()) {
-			if (!r.pending) {
-				if (++g_ring_pollers <= kRingPollers) poll_for(kRingPollUs, has_work);
-				--g_ring_pollers;
-			}
-			std::unique_lock<std::mutex> g(r.lock);
-			r.sleeping = true;
-			if (r.pending)
-				idle = !r.cv.wait_for(g, std::chrono::microseconds(500), has_work);
-			else
-				r.cv.wait(g, has_work);
-			r.sleeping = false;
-		}
-		const uint64_t at = r.read_count;
-		size_t n = (size_t)(r.write_count - at);
-		if (!idle && n == 0) break;  // stop requested, ring empty
-		{
-			std::lock_guard<std::mutex> g(p->lock);
-			if (idle) {
-				if (!p->hold.load()) (void)submit_pending(*p);
-			} else
-				n = run_ring(*p, r.words.get(), at, n, local.data());
-			r.pending = !p->fe.completed().empty() && !p->hold.load();
-		}
-		if (idle) continue;
-		r.read_count += n;
-		if (r.waiters) {
-			std::lock_guard<std::mutex> g(r.lock);
-			r.progress.notify_all();
-		}
+	size_t decode(const uint32_t *w, size_t n, bool &pending)
+	{
+		std::lock_guard<std::mutex> g(p.lock);
+		n = run_commands(p, w, n);
+		pending = !p.fe.completed().empty() && !p.hold.load();
+		return n;
 	}
-}
-
-// Waits until the ring thread has come as far as `reached` asks.
-template <typename Pred>
-static void ring_wait(CommandRing &r, Pred reached)
-{
-	if (poll_for(kWaitPollUs, reached)) return;
-	std::unique_lock<std::mutex> g(r.lock);
-	r.waiters++;
-	r.progress.wait(g, reached);
-	r.waiters--;
-}
+	void idle(bool &pending)
+	{
+		std::lock_guard<std::mutex> g(p.lock);
+		if (!p.hold.load()) (void)submit_pending(p);
+		pending = !p.fe.completed().empty() && !p.hold.load();
+	}
+};
 
 static CommandRing &ensure_ring(Processor &p)
 {
 	std::lock_guard<std::mutex> g(p.ring_create);
 	if (!p.ring) {
 		p.ring.reset(new CommandRing());
-		p.ring->thr = std::thread(ring_loop, &p);
+		CommandRing *r = p.ring.get();
+		r->start([r, &p] { r->run(RingSink{ p }); });
 	}
 	return *p.ring;
 }
 
-// Copy complete commands (n <= kRingWords words) into the ring.
-static void ring_push(Processor &p, const uint32_t *w, size_t n)
-{
-	CommandRing &r = ensure_ring(p);
-	std::lock_guard<std::mutex> pg(r.push_lock);
-	if (r.write_count + n > r.read_count + kRingWords)
-		ring_wait(r, [&] { return r.write_count + n <= r.read_count + kRingWords; });
-	const size_t pos = (size_t)(r.write_count & (kRingWords - 1)), flat = std::min(n, kRingWords - pos);
-	memcpy(r.words.get() + pos, w, flat * 4);
-	memcpy(r.words.get(), w + flat, (n - flat) * 4);
-	r.write_count += n;
-	if (r.sleeping) {
-		std::lock_guard<std::mutex> g(r.lock);
-		r.cv.notify_one();
-	}
-}
-
-// Wait until the ring thread has decoded everything enqueued so far
-// (CommandRing::drain, command_ring.cpp:63-69).
-static void ring_drain(Processor &p)
-{
-	CommandRing *r;
-	{
-		std::lock_guard<std::mutex> g(p.ring_create);
-		r = p.ring.get();
-	}
-	if (!r) return;
-	const uint64_t end = r->write_count;
-	ring_wait(*r, [&] { return r->read_count >= end; });
-}
-
-// Whether the ring holds commands not decoded yet.
-static bool ring_busy(Processor &p)
-{
-	CommandRing *r;
-	{
-		std::lock_guard<std::mutex> g(p.ring_create);
-		r = p.ring.get();
-	}
-	if (!r) return false;
-	return r->read_count != r->write_count;
-}
-
-static bool has_ring(Processor &p)
+// The ring, or null when nothing has been enqueued yet.
+static CommandRing *ring_of(Processor &p)
 {
 	std::lock_guard<std::mutex> g(p.ring_create);
-	return p.ring != nullptr;
+	return p.ring.get();
+}
+
+static void ring_drain(Processor &p)
+{
+	if (CommandRing *r = ring_of(p)) r->drain();
 }
 
 // Send a meta command in-band when the processor has a ring, else run it
 // on the calling thread.
 static void meta_command(Processor &p, const uint32_t *w, size_t n)
 {
-	if (has_ring(p)) {
-		ring_push(p, w, n);
+	if (CommandRing *r = ring_of(p)) {
+		r->push(w, n);
 		return;
 	}
 	std::lock_guard<std::mutex> g(p.lock);
 	run_commands(p, w, n);
-}
-
-static void stop_ring(Processor &p)
-{
-	CommandRing *r;
-	{
-		std::lock_guard<std::mutex> g(p.ring_create);
-		r = p.ring.get();
-	}
-	if (!r) return;
-	{
-		std::lock_guard<std::mutex> g(r->lock);
-		r->stop = true;
-		r->cv.notify_all();
-	}
-	if (r->thr.joinable()) r->thr.join();
 }
 
 // A recorded submission: device-resident inputs and scratch for a fixed set
@@ -2379,7 +2224,7 @@ void rdp_mi_destroy(rdp_mi_processor *h)
 	rdp_mi_idle(h);
 	Processor &p = h->p;
 	if (p.dump) p.dump->close();
-	stop_ring(p);
+	if (CommandRing *r = ring_of(p)) r->finish();
 	p.vi.release();
 	(void)coherent_complete(p);
 	(void)hipFree(p.d_rdram);
@@ -2448,7 +2293,7 @@ void rdp_mi_enqueue_command(rdp_mi_processor *h, unsigned num_words, const uint3
 	unsigned len = Frontend::command_length(words[0]);
 	if (len == 0 || len > num_words) return;
 	if (h->p.dump) dump_command(h, words, len, true);
-	ring_push(h->p, words, len);
+	ensure_ring(h->p).push(words, len);
 	if (h->p.dump) dump_command(h, words, len, false);
 }
 
@@ -2476,7 +2321,7 @@ size_t rdp_mi_enqueue_command_list(rdp_mi_processor *h, size_t num_words, const 
 	while (i < num_words) {
 		unsigned len = Frontend::command_length(words[i]);
 		if (len == 0 || i + len > num_words || i + len - start > kRingChunk) {
-			if (i > start) ring_push(h->p, words + start, i - start);
+			if (i > start) ensure_ring(h->p).push(words + start, i - start);
 			if (len != 0 && i + len > num_words) return i;
 			if (len == 0) i++;
 			start = i;
@@ -2484,7 +2329,7 @@ size_t rdp_mi_enqueue_command_list(rdp_mi_processor *h, size_t num_words, const 
 		}
 		i += len;
 	}
-	if (i > start) ring_push(h->p, words + start, i - start);
+	if (i > start) ensure_ring(h->p).push(words + start, i - start);
 	return i;
 }
 
@@ -2684,10 +2529,11 @@ static int scanout_queue(Processor &p, const rdp_mi_scanout_options &opts, uint3
 		std::lock_guard<std::mutex> g(p.lock);
 		failed_before = p.submit_error;
 	}
-	if (ring_busy(p)) {
+	CommandRing *r = ring_of(p);
+	if (r && r->busy()) {
 		const uint32_t w[1] = { kMetaFlush << 24 };
-		ring_push(p, w, 1);
-		ring_drain(p);
+		r->push(w, 1);
+		r->drain();
 	}
 	std::lock_guard<std::mutex> g(p.lock);
 	if (int err = flush_now(p)) return err;
