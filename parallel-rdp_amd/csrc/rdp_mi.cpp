@@ -331,9 +331,7 @@ struct Processor {
 	std::atomic<uint64_t> timeline_done{ 0 };  // changed under tl_lock
 	int timeline_error = 0;
 	std::string timeline_error_msg;
-	// The first failed submission of the processor and its message.
-	int submit_error = 0;
-	std::string submit_error_msg;
+	SubmitLog submit_log;
 
 	// RDPDUMP2 capture of everything sent through rdp_mi_enqueue_command,
 	// the VI registers and scanouts (rdp_device.cpp:60-73, 874-897, 970-975,
@@ -1549,12 +1547,7 @@ static int submit_pending(Processor &p)
 	std::lock_guard<std::mutex> g(c.lock);
 	Processor *pp = &p;
 	const int err = submit_processors(&pp, 1, false);
-	// A failed submission from the ring thread (idle or pass-count submits)
-	// is reported by the next timeline signal, with its message.
-	if (err && !p.submit_error) {
-		p.submit_error = err;
-		p.submit_error_msg = g_last_error;
-	}
+	if (err) p.submit_log.failed(err, g_last_error);
 	return err;
 }
 
@@ -1571,11 +1564,11 @@ static int flush_now(Processor &p)
 static void signal_now(Processor &p, uint64_t value)
 {
 	const int err = flush_now(p);
-	if (p.submit_error) {
+	if (p.submit_log.first) {
 		std::lock_guard<std::mutex> g(p.tl_lock);
 		if (!p.timeline_error) {
-			p.timeline_error = p.submit_error;
-			p.timeline_error_msg = p.submit_error_msg;
+			p.timeline_error = p.submit_log.first;
+			p.timeline_error_msg = p.submit_log.first_msg;
 		}
 	}
 	Context &c = ctx();
@@ -2522,22 +2515,9 @@ void rdp_mi_scanout_options_default(rdp_mi_scanout_options *o)
 static int scanout_queue(Processor &p, const rdp_mi_scanout_options &opts, uint32_t *out, unsigned *width,
                          unsigned *height, hipEvent_t done)
 {
-	// A ring thread still decoding submits its own passes, with their words in
-	// its core's caches.
-	int failed_before;
-	{
-		std::lock_guard<std::mutex> g(p.lock);
-		failed_before = p.submit_error;
-	}
-	CommandRing *r = ring_of(p);
-	if (r && r->busy()) {
-		const uint32_t w[1] = { kMetaFlush << 24 };
-		r->push(w, 1);
-		r->drain();
-	}
-	std::lock_guard<std::mutex> g(p.lock);
-	if (int err = flush_now(p)) return err;
-	if (p.submit_error && !failed_before) return set_error(p.submit_error, "%s", p.submit_error_msg.c_str());
+	std::unique_lock<std::mutex> g(p.lock, std::defer_lock);
+	if (int err = flush_ring(ring_of(p), g, p.submit_log, [&p] { return flush_now(p); }))
+		return set_error(err, "%s", p.submit_log.last_msg.c_str());
 	Context &c = ctx();
 	std::lock_guard<std::mutex> lg(c.lock);
 	if (p.coherent) {

@@ -18,6 +18,7 @@
 #include <condition_variable>
 #include <memory>
 #include <mutex>
+#include <string>
 #include <thread>
 #include <vector>
 
@@ -174,5 +175,46 @@ private:
 	std::thread thr;
 	std::atomic<bool> stop{ false };
 };
+
+// A processor's failed submissions (under its lock).  The ring thread's have no
+// caller to return to: the first one's code and message go to the next timeline
+// signal; the count and the last one's tell a caller whether one failed since it
+// last looked.
+struct SubmitLog {
+	int first = 0, last = 0;
+	std::string first_msg, last_msg;
+	uint64_t failures = 0;
+
+	void failed(int err, const std::string &msg)
+	{
+		if (!first) {
+			first = err;
+			first_msg = msg;
+		}
+		last = err;
+		last_msg = msg;
+		failures++;
+	}
+};
+
+// Submits everything pushed so far and returns 0 or the code of a submission
+// that failed meanwhile, on whichever thread.  A ring thread still decoding submits
+// its own passes, with their words in its core's caches; `flush` does it
+// otherwise.  g holds the processor's lock on return.
+template <typename Flush>
+int flush_ring(CommandRing *ring, std::unique_lock<std::mutex> &g, const SubmitLog &log, Flush flush)
+{
+	g.lock();
+	const uint64_t seen = log.failures;
+	g.unlock();
+	if (ring && ring->busy()) {
+		const uint32_t w[1] = { kMetaFlush << 24 };
+		ring->push(w, 1);
+		ring->drain();
+	}
+	g.lock();
+	if (int err = flush()) return err;
+	return log.failures != seen ? log.last : 0;
+}
 
 }  // namespace rdp_mi

@@ -90,7 +90,8 @@ void produce(CommandRing &r, uint32_t who, uint32_t count, size_t most, uint32_t
 int fail(const char *what)
 {
 	printf("%s\n", what);
-	return 1;
+	fflush(stdout);
+	_Exit(1);  // threads may still run
 }
 
 int check(const Sink &s, const uint32_t *counts, int producers)
@@ -162,6 +163,52 @@ int main(int argc, char **argv)
 		if (count > 8 && !s.idles) return fail("no idle call");
 		if (s.held) return fail("work left waiting");
 		return check(s, counts, 1);
+	}
+	if (mode == 4) {
+		// Submissions that fail, by the ring thread while it decodes or by the caller:
+		// each flush reports its own, and one that works reports none.
+		r.finish();
+		struct Failing {
+			std::mutex &lock;
+			SubmitLog &log;
+			std::atomic<int> &code;
+			size_t decode(const uint32_t *w, size_t n, bool &pending)
+			{
+				std::this_thread::sleep_for(std::chrono::milliseconds(20));
+				std::lock_guard<std::mutex> g(lock);
+				for (size_t i = 0; i < n; i++)
+					if (w[i] == kMetaFlush << 24 && code) log.failed(code, "ring");
+				pending = false;
+				return n;
+			}
+			void idle(bool &) {}
+		};
+		CommandRing q;
+		std::mutex lock;
+		SubmitLog log;
+		std::atomic<int> code{ 0 };
+		q.start([&] { q.run(Failing{ lock, log, code }); });
+		const uint32_t w[1] = { 0 };
+		const int codes[] = { 0, -3, -3, 0, -5, 0, 0, -3 };
+		for (int want : codes) {
+			code = want;
+			q.push(w, 1);  // the ring thread is busy for 20 ms
+			std::unique_lock<std::mutex> g(lock, std::defer_lock);
+			const int got = flush_ring(&q, g, log, [] { return 0; });
+			if (got != want || !g.owns_lock()) return fail("a failure on the ring thread is lost or made up");
+		}
+		for (int want : codes) {  // the ring is empty: the caller submits
+			std::unique_lock<std::mutex> g(lock, std::defer_lock);
+			const int got = flush_ring(want == -5 ? nullptr : &q, g, log, [&] {
+				if (want) log.failed(want, "caller");
+				return want;
+			});
+			if (got != want || !g.owns_lock()) return fail("a failure of the caller's own flush is lost or made up");
+		}
+		q.finish();
+		if (log.first != -3 || log.first_msg != "ring" || log.last_msg != "caller" || log.failures != 8) return fail("the log");
+		printf("ok\n");
+		return 0;
 	}
 	return fail("unknown mode");
 }
