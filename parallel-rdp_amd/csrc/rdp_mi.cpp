@@ -329,7 +329,7 @@ struct Processor {
 	std::mutex tl_lock;
 	std::condition_variable tl_cv;
 	std::atomic<uint64_t> timeline_done{ 0 };  // changed under tl_lock
-	int timeline_error = 0;
+	std::atomic<int> timeline_error{ 0 };      // the same
 	std::string timeline_error_msg;
 	SubmitLog submit_log;
 
@@ -2360,12 +2360,8 @@ int rdp_mi_wait_for_timeline_timeout(rdp_mi_processor *h, uint64_t value, uint64
 {
 	if (!h) return set_error(RDP_MI_ERROR_INVALID_ARGUMENT, "null processor");
 	Processor &p = h->p;
-	if (timeout_us >= (uint64_t)kWaitPollUs) poll_for(kWaitPollUs, [&] { return p.timeline_done >= value; });
-	std::unique_lock<std::mutex> g(p.tl_lock);
-	auto ready = [&] { return p.timeline_done >= value || p.timeline_error != 0; };
-	if (timeout_us == UINT64_MAX)
-		p.tl_cv.wait(g, ready);
-	else if (!p.tl_cv.wait_for(g, std::chrono::microseconds((int64_t)std::min<uint64_t>(timeout_us, 1ull << 50)), ready))
+	std::unique_lock<std::mutex> g(p.tl_lock, std::defer_lock);
+	if (!wait_ready(g, p.tl_cv, timeout_us, [&] { return p.timeline_done >= value || p.timeline_error != 0; }))
 		return set_error(RDP_MI_ERROR_TIMEOUT, "timeline value %llu not reached within %llu us",
 		                 (unsigned long long)value, (unsigned long long)timeout_us);
 	if (p.timeline_error)

@@ -34,12 +34,12 @@ constexpr size_t kRingChunk = 1u << 12;
 
 // Waits for something another thread or the GPU finishes within a frame poll
 // before they sleep: waking a thread whose core has gone idle took 50 us and more
-// here, two or three times a frame.  Callers poll for kWaitPollUs; a ring thread
-// without work for kRingPollUs, and only kRingPollers of them at a time, so that
-// many processors do not keep every core busy.
+// here, two or three times a frame.  Callers poll for kWaitPollUs, a ring thread
+// without work for kRingPollUs; only kWaitPollers and kRingPollers of them at a
+// time, so that many processors do not keep every core busy.
 constexpr int64_t kWaitPollUs = 1000, kRingPollUs = 400;
-constexpr int kRingPollers = 2;
-inline std::atomic<int> g_ring_pollers{ 0 };
+constexpr int kWaitPollers = 4, kRingPollers = 2;
+inline std::atomic<int> g_wait_pollers{ 0 }, g_ring_pollers{ 0 };
 template <typename Pred>
 bool poll_for(int64_t us, Pred done)
 {
@@ -51,6 +51,31 @@ bool poll_for(int64_t us, Pred done)
 		}
 		if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(us)) return false;
 	}
+}
+
+// The same where fewer than `most` threads poll already; otherwise one look.
+template <typename Pred>
+bool poll_among(std::atomic<int> &pollers, int most, int64_t us, Pred done)
+{
+	const bool polls = ++pollers <= most;
+	const bool ok = polls ? poll_for(us, done) : done();
+	--pollers;
+	return ok;
+}
+
+// Waits for `ready` (atomics changed under g's mutex, announced through cv) for
+// timeout_us at most, the time it polls included; UINT64_MAX: as long as it takes.
+// g holds its mutex on return.
+template <typename Ready>
+bool wait_ready(std::unique_lock<std::mutex> &g, std::condition_variable &cv, uint64_t timeout_us, Ready ready)
+{
+	const auto start = std::chrono::steady_clock::now();
+	const int64_t us = (int64_t)std::min<uint64_t>(timeout_us, 1ull << 50);
+	poll_among(g_wait_pollers, kWaitPollers, std::min(us, kWaitPollUs), ready);
+	g.lock();
+	if (timeout_us != UINT64_MAX) return cv.wait_until(g, start + std::chrono::microseconds(us), ready);
+	cv.wait(g, ready);
+	return true;
 }
 
 class CommandRing {
@@ -97,10 +122,7 @@ public:
 		for (;;) {
 			bool idle = false;
 			if (!has_work()) {
-				if (!pending) {
-					if (++g_ring_pollers <= kRingPollers) poll_for(kRingPollUs, has_work);
-					--g_ring_pollers;
-				}
+				if (!pending) poll_among(g_ring_pollers, kRingPollers, kRingPollUs, has_work);
 				std::unique_lock<std::mutex> g(lock);
 				sleeping = true;
 				if (pending)
@@ -152,7 +174,7 @@ private:
 	template <typename Pred>
 	void wait_for(Pred reached)
 	{
-		if (poll_for(kWaitPollUs, reached)) return;
+		if (poll_among(g_wait_pollers, kWaitPollers, kWaitPollUs, reached)) return;
 		std::unique_lock<std::mutex> g(lock);
 		waiters++;
 		progress.wait(g, reached);

@@ -210,5 +210,52 @@ int main(int argc, char **argv)
 		printf("ok\n");
 		return 0;
 	}
+	if (mode == 5) {
+		// Timed waits end at their timeout, the polled time included (the shortest of
+		// ten: another thread may hold the core), and at once when what they wait for
+		// or an error is there.
+		r.finish();
+		std::mutex m;
+		std::condition_variable cv;
+		std::atomic<uint64_t> done{ 0 };
+		std::atomic<int> error{ 0 };
+		auto ready = [&] { return done >= 1 || error != 0; };
+		auto timed = [&](uint64_t us, bool want) {
+			int64_t best = INT64_MAX;
+			for (int i = 0; i < 10; i++) {
+				const auto t0 = std::chrono::steady_clock::now();
+				std::unique_lock<std::mutex> g(m, std::defer_lock);
+				if (wait_ready(g, cv, us, ready) != want || !g.owns_lock()) fail("the wrong answer");
+				const auto t = std::chrono::steady_clock::now() - t0;
+				best = std::min<int64_t>(best, std::chrono::duration_cast<std::chrono::microseconds>(t).count());
+			}
+			return best;
+		};
+		for (uint64_t us : { 0ull, 300ull, 1000ull, 1500ull, 4000ull }) {
+			const int64_t t = timed(us, false);
+			if (t < (int64_t)us) return fail("a wait ended early");
+			if (t > (int64_t)us + 700) return fail("a wait overran its timeout");
+		}
+		error = -3;
+		if (timed(UINT64_MAX, true) > 300) return fail("an error is there and the wait goes on");
+		error = 0;
+		std::thread late([&] {
+			std::this_thread::sleep_for(std::chrono::milliseconds(30));
+			std::lock_guard<std::mutex> g(m);
+			done = 1;
+			cv.notify_all();
+		});
+		std::vector<std::thread> others;  // more waiters than may poll
+		for (int i = 0; i < 12; i++)
+			others.emplace_back([&] {
+				std::unique_lock<std::mutex> g(m, std::defer_lock);
+				if (!wait_ready(g, cv, UINT64_MAX, ready)) fail("the wrong answer");
+			});
+		late.join();
+		for (auto &t : others) t.join();
+		if (g_wait_pollers != 0) return fail("pollers left");
+		printf("ok\n");
+		return 0;
+	}
 	return fail("unknown mode");
 }

@@ -2,8 +2,9 @@
 the CPU, plain and under ThreadSanitizer: two producers with a thread that
 drains, a full ring whose producers go to sleep, wrap-around in the middle of a
 command, an end with commands left, and pauses around the polling times; and that
-every failed submission is reported by the flush it belongs to.  A lost wake-up
-hangs the probe and fails by its time limit."""
+every failed submission is reported by the flush it belongs to, and timed waits
+end at their timeout.  A lost
+wake-up hangs the probe and fails by its time limit."""
 import os
 import subprocess
 
@@ -21,7 +22,7 @@ def probe(request, tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("mode,count", [(0, 20000), (1, 12000), (2, 6000), (3, 200), (2, 1), (0, 1), (4, 0)])
+@pytest.mark.parametrize("mode,count", [(0, 20000), (1, 12000), (2, 6000), (3, 200), (2, 1), (0, 1), (4, 0), (5, 0)])
 def test_ring(probe, mode, count):
     run = subprocess.run([probe, str(mode), str(count)], capture_output=True, text=True, timeout=100)
     assert run.returncode == 0 and run.stdout.strip() == "ok", run.stdout + run.stderr[-3000:]
