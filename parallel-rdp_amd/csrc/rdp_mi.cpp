@@ -33,6 +33,7 @@
 #include "rdp_digest.hpp"
 #include "rdp_dump.hpp"
 #include "rdp_frontend.hpp"
+#include "rdp_groups.hpp"
 #include "rdp_hazard.hpp"
 #include "rdp_ring.hpp"
 #include "rdp_types.hpp"
@@ -778,12 +779,6 @@ static int execute_launches(const std::vector<Launch> &launches, Lane &lane, con
 	return 0;
 }
 
-// Limits of a group of rounds that share setup launches: scratch (a frame of
-// 8192 small triangles takes about 25 MB) and the 15 bits of a work item's pass
-// index.
-constexpr size_t kGroupScratchBytes = 64u << 20;
-constexpr uint32_t kGroupMaxPasses = 1u << 12;
-
 // From this size on a serving lane's packed inputs go through the copy engine: the
 // upload kernel's waves would take slots on the GPU from the other lanes' rasters
 // for as long as PCIe takes (3 lanes at 40000 frames/s, batches of 5 to 9 frames
@@ -832,10 +827,7 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 	// Submissions with a round of many passes run every round's setup and
 	// binning ahead on the lane's prep stream (execute_launches), so each
 	// round keeps its own scratch region and is a group of its own.  Otherwise
-	// rounds run in series: consecutive rounds form a group while their scratch
-	// stays within kGroupScratchBytes, and groups share one region.  An
-	// upscaled pass reads the TMEM snapshots its native pass (the round before)
-	// left in that round's scratch, so it never begins a group.
+	// rounds run in series, and consecutive ones form groups (GroupWalk).
 	bool upscaled = false;
 	size_t widest = 0;
 	for (const auto &round : rounds) {
@@ -845,7 +837,9 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 	const bool prep_ahead = widest >= kOverlapMinPasses;
 	const LaunchPlan plan = launch_plan(rounds.size(), widest, upscaled);
 	uint32_t num_passes = 0;
-	size_t off = 0, max_scratch = 0, scratch_base = 0;
+	size_t off = 0, max_scratch = 0;
+	GroupWalk walk;
+	walk.own = prep_ahead;
 	for (size_t r = 0; r < rounds.size(); r++) {
 		// Work items carry the pass index above 17 bits of per-pass index.
 		if (rounds[r].size() > (1u << 15))
@@ -858,25 +852,20 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 		for (uint32_t c = 0; c < kRasterClasses; c++) L.n_raster_class[c] = L.n_quad_class[c] = L.n_up_class[c] = 0;
 		pl[r].resize(rounds[r].size());
 		size_t round_scratch = 0;
-		bool joins = false;  // an upscaled pass: in its native pass's group
+		bool upscaled_round = false;
 		for (size_t i = 0; i < rounds[r].size(); i++) {
 			pl[r][i].sl = scratch_layout(*rounds[r][i].pass);
 			round_scratch += pl[r][i].sl.total;
-			joins = joins || rounds[r][i].pass->scale_log2 != 0;
+			upscaled_round = upscaled_round || rounds[r][i].pass->scale_log2 != 0;
 		}
-		const bool fits = !groups.empty() && scratch_base + round_scratch <= kGroupScratchBytes &&
-		                  num_passes - rl[groups.back().first].first_pass <= kGroupMaxPasses;
-		if (prep_ahead || r == 0 || !(joins || fits)) {
-			groups.push_back({ r, 0, !prep_ahead });
-			if (!prep_ahead) scratch_base = 0;
-		}
+		if (walk.next((uint32_t)rounds[r].size(), round_scratch, upscaled_round)) groups.push_back({ r, 0, !prep_ahead });
 		Group &G = groups.back();
 		L.group = (uint32_t)groups.size() - 1;
 		// Shared TMEM replay: every upload of the group may run before every
 		// raster of it.
 		for (size_t q = G.first; q < r && G.tmem; q++) G.tmem = tmem_may_start_before(rounds, r, q);
 		G.rounds++;
-		size_t scr = scratch_base;
+		size_t scr = walk.scratch;
 		for (size_t i = 0; i < rounds[r].size(); i++) {
 			const HostPass &hp = *rounds[r][i].pass;
 			const uint32_t tx = (hp.fb_width + 7) / 8, ty = (hp.fb_height + 7) / 8;
@@ -919,7 +908,7 @@ static int prepare_rounds(Lane &c, const std::vector<std::vector<PassRef>> &roun
 			scr += pi.sl.total;
 		}
 		max_scratch = std::max(max_scratch, scr);
-		scratch_base = align_up(scr, 256);
+		walk.scratch = align_up(scr, 256);
 		L.items_raster = off;
 		off = align_up(off + (L.n_raster + L.n_fill + L.n_quad) * 4ull, 256);
 		L.items_domain = off;
