@@ -1,6 +1,7 @@
-// Host-side bounds for ordering a round's TMEM replay against the previous
-// round's raster: what a pass's raster can write and what a TMEM upload can
-// read, as RDRAM byte ranges.
+// Host-side bounds of what a pass's raster can write, what a TMEM upload can read
+// and what a clear overwrites whole, as RDRAM byte ranges.  They decide whether a
+// round's TMEM replay may run before the rasters of earlier rounds, and with
+// host-coherent RDRAM which of the caller's pages a submission copies in.
 #pragma once
 
 #include <stdint.h>

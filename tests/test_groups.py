@@ -1,7 +1,8 @@
 """Groups of rounds (parallel-rdp_amd/csrc/rdp_groups.hpp) on the CPU: the index of
 a pass in its group fits the 15 bits a work item has for it however many rounds
 hold an upscaled pass, an upscaled pass's round leaves the scratch of the round
-before it alone, and rounds of one group never share scratch."""
+before it alone, rounds of one group never share scratch, and a group has few
+enough rounds to compare each with all before it."""
 import os
 import random
 import subprocess
@@ -9,7 +10,7 @@ import subprocess
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-PASS_BITS, SCRATCH = 15, 64 << 20
+PASS_BITS, SCRATCH, MOST_ROUNDS = 15, 64 << 20, 64
 
 
 @pytest.fixture(scope="module")
@@ -33,17 +34,22 @@ def rounds_of(kind):
         return [(rng.randint(1, 7), rng.randint(1, 30 << 20), False) for _ in range(3000)]
     if kind == "large":
         return [(1, 40 << 20, k % 2 == 1) for k in range(200)]
+    if kind == "small":
+        return [(2, 12288, False)] * 2000
     return [(rng.randint(1, 7), rng.randint(1, 4 << 20), rng.random() < 0.5 and k > 0) for k in range(6000)]
 
 
-@pytest.mark.parametrize("kind", ["upscaled", "native", "large", "mixed"])
+@pytest.mark.parametrize("kind", ["upscaled", "native", "large", "small", "mixed"])
 def test_groups(probe, kind):
     rounds = rounds_of(kind)
     out = walk(probe, rounds)
     assert len(out) == len(rounds) and out[0][0] == 1
     end = 0  # of the scratch of the round before
+    length = 0  # rounds of the group
     for k, ((passes, scratch, upscaled), (begins, base, total)) in enumerate(zip(rounds, out)):
         assert total <= 1 << PASS_BITS, k
+        length = 1 if begins else length + 1
+        assert length <= MOST_ROUNDS, k
         if upscaled or not begins:
             assert base == end, k
         else:
