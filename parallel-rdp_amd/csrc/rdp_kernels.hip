@@ -13,6 +13,8 @@
 //   k_bin     one wave64 per (tile row, group of 64 primitives), eight per
 //             workgroup: an XOR prefix over the tile columns produces the ordered
 //             64-bit primitive masks.
+//             Beside rasters the same work runs as k_setup, k_span, k_tmem_gather,
+//             k_tmem_scan and k_bin_wave, in blocks that fit between raster waves.
 //   k_raster  one wave64 per 8x8 screen tile: colour/depth/coverage of the 64
 //             pixels live in registers while every binned primitive is shaded
 //             (coverage, interpolation, texturing, combiner) and merged (Z test,
